@@ -72,15 +72,22 @@ __device__ __forceinline__ float gelu(float v) {
 // Bias epilogue of cpu_gemm (math.cpp:431-433): out[f] += beta * c[f % c_size],
 // then optionally a fused Relu (activation.cpp:45-60: std::max(0.0f, v), which
 // is (0 < v) ? v : +0, so -0 and NaN give +0) or Gelu (activation.cpp:239-259).
-__device__ __forceinline__ float bias_add(float v, int64_t f, const float* __restrict__ bias,
-                                          int64_t c_size, float beta, int act) {
-    if (bias != nullptr) {
-        const float t = beta * bias[f % c_size];
-        v = v + t;
-    }
+__device__ __forceinline__ float activate(float v, int act) {
     if (act == PFR_ACT_RELU) v = (0.0f < v) ? v : 0.0f;
     else if (act == PFR_ACT_GELU) v = pfr::gelu(v);
     return v;
+}
+// The same with the output's bias element given (null: none).
+__device__ __forceinline__ float bias_add_at(float v, const float* __restrict__ c, float beta, int act) {
+    if (c != nullptr) {
+        const float t = beta * *c;
+        v = v + t;
+    }
+    return activate(v, act);
+}
+__device__ __forceinline__ float bias_add(float v, int64_t f, const float* __restrict__ bias,
+                                          int64_t c_size, float beta, int act) {
+    return bias_add_at(v, bias != nullptr ? bias + f % c_size : nullptr, beta, act);
 }
 
 // Grow-only device buffer owned by a context.

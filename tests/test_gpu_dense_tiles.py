@@ -1,0 +1,57 @@
+"""The dense strict product over its four workgroup tiles (32 x 32, 64 x 32,
+64 x 64 and 128 x 64 outputs), at the edges of the tiles and of the k chunks
+(32 or 64), with the operands' rows aligned and not, padded leading
+dimensions and both orientations of A.
+
+Bar: bit for bit the oracle's cpu_gemm (math.cpp:377-438), denormal products
+included; NaN where it has NaN."""
+import numpy as np
+import pytest
+
+from oracle import oracle as O
+from pyflamert_amd import rocm
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def ctx():
+    c = rocm.Context(0)
+    yield c
+    c.close()
+
+
+@pytest.mark.parametrize("M,K,N", [
+    # 32 x 32 tiles: K around its chunk of 64 and down to 1
+    (1, 1, 33), (31, 3, 1), (33, 63, 65), (32, 64, 32), (65, 65, 31), (5, 129, 200), (40, 68, 7),
+    # 64 x 32, 64 x 64 and 128 x 64 tiles (chunk 32), one row and column past them
+    (513, 33, 3072), (512, 32, 3041), (1024, 31, 3073), (1025, 36, 3072), (4096, 65, 2047), (4097, 4, 2048)])
+def test_dense_tiles_bit_exact(ctx, M, K, N):
+    import torch
+
+    rng = np.random.default_rng(M + 7 * K + 13 * N)
+    B = rng.standard_normal((K, N)).astype(np.float32)
+    Cb = rng.standard_normal(N).astype(np.float32)
+    for ta in (0, 1):
+        A = rng.standard_normal((K, M) if ta else (M, K)).astype(np.float32)
+        A.flat[::5] *= np.float32(1e-30)  # products down among the denormals
+        A.flat[1::97] = np.float32(1e-41)
+        A.flat[::1013] = np.inf
+        print(f"dense tiles M={M} K={K} N={N} transA={ta}", flush=True)
+        for alpha, C_ in ((1.0, Cb), (-0.75, Cb[:min(N, 7)])):
+            R = O.orc_gemm(A, B * np.float32(1e-9), C_, alpha, 1.5, ta, 0)
+            ldb, ldy = N + 3, N + 1
+            dA = torch.from_numpy(A).cuda()
+            dB = torch.full((K, ldb), float("nan"), device="cuda")
+            dB[:, :N] = torch.from_numpy(B * np.float32(1e-9)).cuda()
+            dC = torch.from_numpy(np.ascontiguousarray(C_)).cuda()
+            dY = torch.full((M, ldy), 7.0, device="cuda")
+            torch.cuda.synchronize()
+            ctx.gemm_dense_dev(dA.data_ptr(), M, K, dB.data_ptr(), N, dY.data_ptr(), transA=ta, alpha=alpha,
+                               beta=1.5, C_ptr=dC.data_ptr(), c_size=C_.size, ldb=ldb, ldy=ldy)
+            ctx.synchronize()
+            Y = dY.cpu().numpy()
+            assert (Y[:, N:] == 7.0).all()
+            nan = np.isnan(R)
+            assert np.array_equal(np.isnan(Y[:, :N]), nan)
+            assert np.array_equal(Y[:, :N].view(np.uint32)[~nan], R.view(np.uint32)[~nan]), (ta, alpha)
