@@ -1057,6 +1057,225 @@ __global__ __launch_bounds__(kI8Threads, 1) void k_sp24_bf16p(int nkt, const v4i
         }
 }
 
+// 2:4 GEMM for few columns or few tiles: the large-tile kernels above own 256 x
+// 128 outputs per workgroup, so a decode batch (8 columns of a 4096-row
+// weight) ran on 16 of 256 CUs and took 45 us for a 28 MB weight.  Here a
+// workgroup owns 16 RB x 16 NB outputs and its W waves split K: wave w takes
+// the steps w, w + W, ... (128 bytes of an XT row each: 128 k of int8, 64 of
+// bf16), so every CU streams its own part of the weight, and the waves' sums
+// meet in LDS once at the end (int32: exact; float: added in wave order).
+// Nothing is shared between the waves before that, so there is no barrier in
+// the loop.  Each wave loads its packed values (the MFMA's lane order) and
+// positions, and the step's XT rows as whole 128-byte lines (lane l: piece l
+// % 8 of row l / 8 and of the row 8 below), into a ring of D register slots,
+// D - 1 steps ahead; the rows pass through 2 NB KiB of LDS of the wave's own
+// into fragment order (16-byte piece p of row r at p ^ ((r >> 1) & 7); LDS
+// operations of a wave run in order, so one buffer serves), a step ahead of
+// the MFMAs where registers allow.  (Fragments loaded straight from XT touch
+// 16 lines per 16 lanes: 4096 x 4096 on 128 rows of activation took 12.5 us
+// instead of 9.0.)  Measured on int8 4096 x 11008 with 8 rows of activation,
+// quantized activation to float output: 55.6 -> 7.0 us, 4.1 TB/s.
+// XT rows past N repeat the last one (never written); XT holds a multiple of
+// 16 bytes per row and pieces past kbytes, whose weights are the packing's
+// zeros, repeat the last one (the bf16 caller's XT is zero-padded to whole
+// steps instead, as 0 * inf is no zero).
+// FLIP: x is uint8, taken as x - 128 (see k_sp24_i8).  Outputs: D's lane holds
+// rows 4 (l / 16) .. + 3 of column l % 16; with `trans` they go to Y[n][m]
+// (the x . W form, 16 bytes per lane), else to Y[m][n].
+struct Sp24Epi {
+    const float* ws;
+    float xs, inv_out;
+    int32_t out_zp;
+    int inrange;
+    int32_t x_zp, zp_shift;
+    const float* xs_dev;
+    const uint8_t* zp_dev;
+    const int32_t* row_sum;
+    int out_kind, trans;
+};
+
+template <bool BF, int RB, int NB, int W, int D, bool FLIP>
+__global__ __launch_bounds__(64 * W) void k_sp24_small(int nsteps, int nkt, const v4i* __restrict__ A,
+                                                       const uint32_t* __restrict__ I, const char* __restrict__ XT,
+                                                       int64_t ldb, int kbytes, int M, int N, int ntn,
+                                                       void* __restrict__ Y, int64_t ldy, Sp24Epi ep) {
+    using Acc = typename std::conditional<BF, v4f, v4i>::type;
+    constexpr int kPart = W * RB * NB * 1024, kRows = W * NB * 2048;
+    __shared__ __attribute__((aligned(1024))) char lds[kPart > kRows ? kPart : kRows];
+    Acc(*const part)[RB * NB][64] = reinterpret_cast<Acc(*)[RB * NB][64]>(lds);  // after the loop
+    const int t = threadIdx.x, w = __builtin_amdgcn_readfirstlane(t >> 6), l = t & 63;
+    const int kb = l >> 4, c = l & 15;
+    int mt, nt;
+    {  // consecutive tiles of the m-major order go to one XCD (they share the weight's rows)
+        const int G = (int)gridDim.x, L = (int)blockIdx.x, xcd = L & 7, slot = L >> 3;
+        const int q = G >> 3, rem = G & 7;
+        const int T = xcd * q + min(xcd, rem) + slot;
+        mt = T / ntn;
+        nt = T % ntn;
+    }
+    const int64_t mb0 = (int64_t)mt * RB;  // the packed rows are padded to 256: every block exists
+    const int n0 = nt * 16 * NB;
+    const v4i* aw[RB];
+    const uint32_t* iw[RB];
+    const char* bw[2 * NB];  // rows 8h + l / 8 of the tile
+#pragma unroll
+    for (int i = 0; i < RB; ++i) {
+        aw[i] = A + (mb0 + i) * nkt * 64 + l;
+        iw[i] = I + (mb0 + i) * (BF ? nkt / 2 : nkt) * 64 + l;
+    }
+#pragma unroll
+    for (int h = 0; h < 2 * NB; ++h) bw[h] = XT + (int64_t)min(n0 + 8 * h + (l >> 3), N - 1) * ldb;
+    char* const rows = lds + w * NB * 2048;
+    // this lane's piece of row 8h + l / 8: the swizzle (row >> 1) & 7 is (4h + l / 16) & 7
+    const int wr = (l >> 3) * 128, wp = l & 7;
+    const int rd = c * 128, rs = (c >> 1) & 7;
+    struct Slot {
+        v4i a[RB], b[2 * NB];
+        uint32_t ix[RB];
+    };
+    auto load = [&](Slot& f, int s) {
+#pragma unroll
+        for (int i = 0; i < RB; ++i) {
+            f.a[i] = aw[i][(int64_t)s * 64];
+            f.ix[i] = iw[i][(int64_t)(BF ? s >> 1 : s) * 64];
+        }
+        const int o = min(128 * s + 16 * wp, kbytes - 16);
+#pragma unroll
+        for (int h = 0; h < 2 * NB; ++h) f.b[h] = *reinterpret_cast<const v4i*>(bw[h] + o);
+        // keep this step's loads ahead of the MFMAs that follow
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    struct Frag {
+        v8i b[NB];
+    };
+    auto arrange = [&](Frag& g, const Slot& f) {
+#pragma unroll
+        for (int h = 0; h < 2 * NB; ++h) {
+            v4i b = f.b[h];
+            if constexpr (FLIP) b ^= (int)0x80808080;
+            *reinterpret_cast<v4i*>(rows + h * 1024 + wr + 16 * (wp ^ ((4 * h + (l >> 4)) & 7))) = b;
+        }
+#pragma unroll
+        for (int j = 0; j < NB; ++j) {
+            const v4i lo = *reinterpret_cast<const v4i*>(rows + j * 2048 + rd + 16 * (kb ^ rs));
+            const v4i hi = *reinterpret_cast<const v4i*>(rows + j * 2048 + rd + 16 * ((4 + kb) ^ rs));
+            g.b[j] = v8i{lo.x, lo.y, lo.z, lo.w, hi.x, hi.y, hi.z, hi.w};
+        }
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    Acc acc[RB][NB];
+#pragma unroll
+    for (int i = 0; i < RB; ++i)
+#pragma unroll
+        for (int j = 0; j < NB; ++j) acc[i][j] = Acc{0, 0, 0, 0};
+    auto mma = [&](const Slot& f, const Frag& g, int s) {
+#pragma unroll
+        for (int j = 0; j < NB; ++j) {
+#pragma unroll
+            for (int i = 0; i < RB; ++i) {
+                if constexpr (BF)
+                    acc[i][j] = __builtin_amdgcn_smfmac_f32_16x16x64_bf16(__builtin_bit_cast(v8bf, f.a[i]),
+                                                                          __builtin_bit_cast(v16bf, g.b[j]), acc[i][j],
+                                                                          (int)(f.ix[i] >> (16 * (s & 1))), 0, 0);
+                else
+                    acc[i][j] = __builtin_amdgcn_smfmac_i32_16x16x128_i8(f.a[i], g.b[j], acc[i][j], (int)f.ix[i], 0, 0);
+            }
+        }
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    const int n = w < nsteps ? (nsteps - w + W - 1) / W : 0;  // this wave's steps
+    if (n > 0) {
+        Slot r[D];
+        Frag g[2];
+        auto step = [&](int i) { return w + W * min(i, n - 1); };
+#pragma unroll
+        for (int u = 0; u + 1 < D; ++u) load(r[u], step(u));
+        constexpr bool AHEAD = D > 2;  // two slots: the other one has only just been asked for
+        if (AHEAD) arrange(g[0], r[0]);
+        int i = 0;
+        static_assert(D % 2 == 0, "the fragment sets alternate");
+        for (; i + D <= n; i += D) {
+#pragma unroll
+            for (int u = 0; u < D; ++u) {
+                load(r[(u + D - 1) % D], step(i + u + D - 1));
+                if (AHEAD) arrange(g[(u + 1) % 2], r[(u + 1) % D]);  // (the last step's: once more)
+                else arrange(g[u % 2], r[u]);
+                mma(r[u], g[u % 2], step(i + u));
+            }
+        }
+#pragma unroll
+        for (int u = 0; u + 1 < D; ++u)
+            if (i + u < n) {
+                if (!AHEAD) arrange(g[u % 2], r[u]);
+                else if (u + 2 < D) arrange(g[(u + 1) % 2], r[u + 1]);
+                mma(r[u], g[u % 2], step(i + u));
+            }
+    }
+    __syncthreads();  // the waves' sums take the place of their rows
+#pragma unroll
+    for (int i = 0; i < RB; ++i)
+#pragma unroll
+        for (int j = 0; j < NB; ++j) part[w][i * NB + j][l] = acc[i][j];
+    __syncthreads();
+    const float xs = BF ? 1.0f : (ep.xs_dev ? *ep.xs_dev : ep.xs);
+    uint32_t zcorr = 0;
+    if constexpr (!BF) zcorr = (uint32_t)((ep.zp_dev ? (int32_t)*ep.zp_dev : ep.x_zp) - ep.zp_shift);
+    for (int e = w; e < RB * NB; e += W) {  // tile e: rows 16 (e / NB), columns 16 (e % NB)
+        Acc v = part[0][e][l];
+#pragma unroll
+        for (int u = 1; u < W; ++u) v += part[u][e][l];
+        const int m = (int)(mb0 + e / NB) * 16 + 4 * kb, col = n0 + 16 * (e % NB) + c;
+        if (col >= N || m >= M) continue;
+        uint32_t out[4];
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            if constexpr (BF) {
+                out[q] = __float_as_uint(v[q]);
+            } else {
+                const int mr = min(m + q, M - 1);
+                const int32_t a = zcorr ? (int32_t)((uint32_t)v[q] - zcorr * (uint32_t)ep.row_sum[mr]) : v[q];
+                if (ep.out_kind == PFR_SP24_OUT_I32) {
+                    out[q] = (uint32_t)a;
+                } else {
+                    const float f = (float)a * (ep.ws[mr] * xs);  // a_scale * b_scale first (quant_ops.cpp:435)
+                    if (ep.out_kind == PFR_SP24_OUT_F32) {
+                        out[q] = __float_as_uint(f);
+                    } else {
+                        const float p = f * ep.inv_out;
+                        int32_t z;
+                        if (ep.inrange && ep.out_zp == 0) {
+                            z = round_clamp_i8<true>(p);
+                        } else {
+                            z = (int32_t)((uint32_t)pfr::f2i_trunc_x86(roundf(p)) + (uint32_t)ep.out_zp);
+                            z = z < -128 ? -128 : (z > 127 ? 127 : z);
+                        }
+                        out[q] = (uint32_t)z;
+                    }
+                }
+            }
+        }
+        if (ep.trans) {
+            uint32_t* yr = static_cast<uint32_t*>(Y) + (int64_t)col * ldy + m;
+            if (m + 3 < M && (ldy & 3) == 0 && (reinterpret_cast<uintptr_t>(Y) & 15) == 0) {
+                *reinterpret_cast<v4i*>(yr) = v4i{(int)out[0], (int)out[1], (int)out[2], (int)out[3]};
+            } else {
+#pragma unroll
+                for (int q = 0; q < 4; ++q)
+                    if (m + q < M) yr[q] = out[q];
+            }
+        } else {
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                if (m + q >= M) continue;
+                if (!BF && ep.out_kind == PFR_SP24_OUT_I8)
+                    static_cast<int8_t*>(Y)[(int64_t)(m + q) * ldy + col] = (int8_t)out[q];
+                else
+                    static_cast<uint32_t*>(Y)[(int64_t)(m + q) * ldy + col] = out[q];
+            }
+        }
+    }
+}
+
 // x - 128 as int8 for uint8 x (K rows of N bytes, ldx apart, to a compact
 // copy): VEC (N and ldx multiples of 16, X 16-byte aligned) flips 16 bytes
 // per thread, otherwise one byte per thread, blockIdx.y striding the rows.
@@ -1418,6 +1637,76 @@ void check_i8(const pfr_sp24* W) {
     if (W->dtype != PFR_I8) throw pfr::Error(PFR_ERR_UNSUPPORTED, "weight is not int8");
 }
 
+// The small-tile kernel's tiles, each with its time in ns: start + workgroups
+// per CU * (each + steps * step).  Fitted to 4096 x {4096, 11008} on 1 .. 512
+// columns with 8 rotating weights (int8, x . W form); for instance 4096 x 4096
+// on 64 columns: 9.9 us in 16 x 16 tiles, 7.7 in 32 x 16, 7.0 in 32 x 32, 8.5
+// in 64 x 32 and 11.8 in 64 x 64; on 512: 57, 43, 43, 28 and 17.
+struct SmallTile {
+    int rb, nb, w, start, each, step;
+};
+constexpr SmallTile kSmallTiles[] = {{1, 1, 8, 3500, 870, 24},
+                                     {2, 1, 8, 3400, 1300, 36},
+                                     {2, 2, 8, 1800, 2400, 87},
+                                     {4, 2, 8, 2500, 3400, 96},
+                                     {4, 4, 4, 6000, 2000, 140}};
+
+// The tile (an index into kSmallTiles) that serves an M x N product of
+// `steps` 128-byte steps soonest, and its time in ns.
+int small_tile(const pfr_ctx* ctx, int64_t M, int64_t N, int64_t steps, int64_t* ns) {
+    int best = 0;
+    *ns = INT64_MAX;
+    for (int i = 0; i < 5; ++i) {
+        const SmallTile& t = kSmallTiles[i];
+        const int64_t wgs = (M + 16 * t.rb - 1) / (16 * t.rb) * ((N + 16 * t.nb - 1) / (16 * t.nb));
+        const int64_t per_cu = (wgs + ctx->num_cu - 1) / ctx->num_cu;
+        const int64_t e = t.start + per_cu * (t.each + steps * t.step);
+        if (e < *ns) *ns = e, best = i;
+    }
+    return best;
+}
+
+// The large-tile kernels' time in ns: a start and so much per 128-byte step
+// and round, more when more tiles share the memory (measured: int8 from
+// row-major X 18.7 us at 16 and 22.8 at 172 tiles, K = 4096; from XT 22 and
+// 29; bf16 29 and 38).  And that of transposing the activation first.
+int64_t large_ns(const pfr_ctx* ctx, const pfr_sp24* W, int64_t N, int64_t steps, bool xrow) {
+    const int64_t tiles = W->Mp / kI8TileM * ((N + kI8TileN - 1) / kI8TileN);
+    const int64_t rounds = (tiles + ctx->num_cu - 1) / ctx->num_cu, busy = std::min<int64_t>(tiles, ctx->num_cu);
+    const int64_t step = W->dtype == PFR_BF16 ? std::min<int64_t>(380 + 9 * busy / 2, 600)
+                                              : (xrow ? 430 + 7 * busy / 10 : 500 + 14 * busy / 10);
+    return 5000 + rounds * steps * step;
+}
+constexpr int64_t kTransposeNs = 4000;
+
+// Launches the small-tile kernel: XT as it describes, Y and ep as set by the
+// caller.
+template <bool BF, bool FLIP>
+void launch_small(pfr_ctx* ctx, const pfr_sp24* W, int tile, const char* XT, int64_t ldb, int64_t kbytes, int64_t N,
+                  void* Y, int64_t ldy, const Sp24Epi& ep) {
+    const int nkt = (int)(W->Kp / (BF ? 64 : 128)), steps = (int)((W->K + (BF ? 63 : 127)) / (BF ? 64 : 128));
+#define PFR_SMALL_TILE(IDX, RBV, NBV, WV, DV)                                                                       \
+    case IDX: {                                                                                                     \
+        static_assert(kSmallTiles[IDX].rb == RBV && kSmallTiles[IDX].nb == NBV && kSmallTiles[IDX].w == WV, "tile"); \
+        const int ntn = (int)((N + 16 * NBV - 1) / (16 * NBV));                                                     \
+        const dim3 grid((unsigned)((W->M + 16 * RBV - 1) / (16 * RBV) * ntn));                                      \
+        hipLaunchKernelGGL((k_sp24_small<BF, RBV, NBV, WV, DV, FLIP>), grid, dim3(64 * WV), 0, ctx->stream, steps,  \
+                           nkt, static_cast<const v4i*>(W->a), W->idx, XT, ldb, (int)kbytes, (int)W->M, (int)N, ntn, \
+                           Y, ldy, ep);                                                                             \
+        break;                                                                                                      \
+    }
+    switch (tile) {
+        PFR_SMALL_TILE(0, 1, 1, 8, 4)
+        PFR_SMALL_TILE(1, 2, 1, 8, 4)
+        PFR_SMALL_TILE(2, 2, 2, 8, 4)
+        PFR_SMALL_TILE(3, 4, 2, 8, 4)
+        default:
+        PFR_SMALL_TILE(4, 4, 4, 4, 2)
+    }
+#undef PFR_SMALL_TILE
+    PFR_HIP(hipGetLastError());
+}
+
 // XT for the activation: int8 or bf16 bits, Np x Kp.
 // x_u8: X holds uint8 values.  x_zp: the activation zero point, or
 // (zp_dev set) a device uint8 holding it; x_scale likewise with xs_dev.
@@ -1448,6 +1737,27 @@ void gemm_i8_dev(pfr_ctx* ctx, const pfr_sp24* W, const int8_t* X, int64_t N, in
             inrange = (double)W->Kp * 8192.0 * (double)W->w_scale_max * (double)x_scale * (double)inv_out <
                       1073741824.0;
     }
+    const int64_t Kp = W->Kp;
+    const bool aligned = ldx % 16 == 0 && (reinterpret_cast<uintptr_t>(X) & 15) == 0;
+    // X itself serves the large tiles when whole 128-column, 128-row B tiles
+    // stay inside it and its rows are 16-byte aligned; otherwise it is
+    // transposed into a zero-padded XT (Np x Kp) first.
+    const bool xrow = W->K == Kp && N % kI8TileN == 0 && (x_u8 || aligned);
+    int64_t small_ns = 0;
+    const int tile = small_tile(ctx, W->M, N, (W->K + 127) / 128, &small_ns);
+    if (small_ns + (xrow ? kTransposeNs : 0) < large_ns(ctx, W, N, Kp / 128, xrow)) {
+        const int64_t rows = round_up(N, 16);
+        int8_t* xt = static_cast<int8_t*>(ctx->scratch[3].ensure((size_t)(rows * Kp)));
+        hipLaunchKernelGGL(k_transpose_i8, dim3((unsigned)(Kp / 64), (unsigned)((rows + 255) / 256)), dim3(256), 0,
+                           ctx->stream, X, W->K, N, ldx, aligned ? 1 : 0, xt, Kp, rows);
+        PFR_HIP(hipGetLastError());
+        const Sp24Epi ep{W->w_scale, x_scale, inv_out, out_zp, inrange, x_zp, x_u8 ? 128 : 0, xs_dev, zp_dev,
+                         W->row_sum, out_kind, 0};
+        const char* b = reinterpret_cast<const char*>(xt);
+        if (x_u8) launch_small<false, true>(ctx, W, tile, b, Kp, Kp, N, Y, ldy, ep);
+        else launch_small<false, false>(ctx, W, tile, b, Kp, Kp, N, Y, ldy, ep);
+        return;
+    }
     if (x_u8) {
         // the signed MFMA takes x - 128; the zero-point correction adds the 128 back
         uint8_t* xs8 = static_cast<uint8_t*>(ctx->scratch[1].ensure((size_t)(W->K * N) + 16));
@@ -1462,15 +1772,9 @@ void gemm_i8_dev(pfr_ctx* ctx, const pfr_sp24* W, const int8_t* X, int64_t N, in
         X = reinterpret_cast<const int8_t*>(xs8);
         ldx = N;
     }
-    const int64_t Kp = W->Kp;
     const int nkt = (int)(Kp / 128);
     const int yvec = (ldy % 16 == 0 && (reinterpret_cast<uintptr_t>(Y) & 15) == 0) ? 1 : 0;
     const v4i* A = static_cast<const v4i*>(W->a);
-    // The kernel reads whole 128-column, 128-row B tiles.  X itself serves
-    // when those stay inside it and its rows are 16-byte aligned; otherwise
-    // it is transposed into a zero-padded XT (Np x Kp) first.
-    const bool xrow = W->K == Kp && N % kI8TileN == 0 && ldx % 16 == 0 &&
-                      (reinterpret_cast<uintptr_t>(X) & 15) == 0;
     int64_t Np = N;
     const int8_t* B = X;
     int64_t ldb = ldx;
@@ -1563,6 +1867,27 @@ void gemm_qt_dev(pfr_ctx* ctx, const pfr_sp24* W, const uint8_t* X, bool x_u8, i
     pfr::require(X != nullptr && Y != nullptr, "null X/Y");
     if (!xs_dev) pfr::require(x_scale > 0.0f && std::isfinite(x_scale), "x_scale must be positive and finite");
     const int64_t Kp = W->Kp, Np = round_up(T, kI8TileN), ldyp = round_up(T, 16);
+    int64_t small_ns = 0;
+    const int tile = small_tile(ctx, W->M, T, (W->K + 127) / 128, &small_ns);
+    if (small_ns < large_ns(ctx, W, T, Kp / 128, false) + 2 * kTransposeNs) {
+        // the rows of X are the K-contiguous operand as they are, when their
+        // 16-byte pieces are whole and aligned
+        const bool direct = W->K >= 16 && W->K % 16 == 0 && ldx % 16 == 0 && (reinterpret_cast<uintptr_t>(X) & 15) == 0;
+        const uint8_t* b = X;
+        if (!direct) {
+            uint8_t* xt = static_cast<uint8_t*>(ctx->scratch[3].ensure((size_t)(T * Kp)));
+            hipLaunchKernelGGL(k_pad_act<false>, dim3((unsigned)((T * Kp + 255) / 256)), dim3(256), 0, ctx->stream, X, T,
+                               W->K, ldx, xt, Kp, T);
+            PFR_HIP(hipGetLastError());
+            b = xt;
+        }
+        const Sp24Epi ep{W->w_scale, x_scale, 1.0f, 0, 0, x_zp, x_u8 ? 128 : 0, xs_dev, zp_dev, W->row_sum,
+                         PFR_SP24_OUT_F32, 1};
+        const char* bc = reinterpret_cast<const char*>(b);
+        if (x_u8) launch_small<false, true>(ctx, W, tile, bc, direct ? ldx : Kp, direct ? W->K : Kp, T, Y, ldy, ep);
+        else launch_small<false, false>(ctx, W, tile, bc, direct ? ldx : Kp, direct ? W->K : Kp, T, Y, ldy, ep);
+        return;
+    }
     uint8_t* xt = static_cast<uint8_t*>(ctx->scratch[3].ensure((size_t)(Np * Kp)));
     float* yp = static_cast<float*>(ctx->scratch[5].ensure((size_t)(W->M * ldyp) * 4));
     const unsigned pb = (unsigned)((Np * Kp + 255) / 256);
@@ -1594,6 +1919,19 @@ void gemm_bf16_dev(pfr_ctx* ctx, const pfr_sp24* W, const uint16_t* X, int64_t N
     // it is transposed into a zero-padded XT (Np x Kp) first.
     const bool xrow = W->K == W->Kp && N % kI8TileN == 0 && ldx % 8 == 0 &&
                       (reinterpret_cast<uintptr_t>(X) & 15) == 0;
+    int64_t small_ns = 0;
+    const int tile = small_tile(ctx, W->M, N, (W->K + 63) / 64, &small_ns);
+    const int vec = (ldx % 4 == 0 && (reinterpret_cast<uintptr_t>(X) & 7) == 0) ? 1 : 0;
+    if (small_ns + (xrow ? kTransposeNs : 0) < large_ns(ctx, W, N, W->Kp / 64, xrow)) {
+        const int64_t rows = round_up(N, 64);
+        uint16_t* xt = static_cast<uint16_t*>(ctx->scratch[3].ensure(sizeof(uint16_t) * (size_t)(rows * W->Kp)));
+        hipLaunchKernelGGL(k_transpose_b16, dim3((unsigned)(W->Kp / 64), (unsigned)(rows / 64)), dim3(256), 0,
+                           ctx->stream, X, W->K, N, ldx, vec, xt, W->Kp);
+        PFR_HIP(hipGetLastError());
+        launch_small<true, false>(ctx, W, tile, reinterpret_cast<const char*>(xt), 2 * W->Kp, 2 * W->Kp, N, Y, ldy,
+                                  Sp24Epi{});
+        return;
+    }
     const int64_t Np = round_up(N, kI8TileN);
     const int ntn = (int)(Np / kI8TileN);
     const dim3 grid((unsigned)(W->Mp / kI8TileM * ntn));
@@ -1602,7 +1940,6 @@ void gemm_bf16_dev(pfr_ctx* ctx, const pfr_sp24* W, const uint16_t* X, int64_t N
                            static_cast<const v4i*>(W->a), W->idx, X, ldx * 2, (int)W->M, (int)N, Y, ldy, ntn);
     } else {
         uint16_t* xt = static_cast<uint16_t*>(ctx->scratch[3].ensure(sizeof(uint16_t) * (size_t)(Np * W->Kp)));
-        const int vec = (ldx % 4 == 0 && (reinterpret_cast<uintptr_t>(X) & 7) == 0) ? 1 : 0;
         hipLaunchKernelGGL(k_transpose_b16, dim3((unsigned)(W->Kp / 64), (unsigned)(Np / 64)), dim3(256), 0,
                            ctx->stream, X, W->K, N, ldx, vec, xt, W->Kp);
         PFR_HIP(hipGetLastError());
