@@ -1079,6 +1079,14 @@ __global__ __launch_bounds__(kI8Threads, 1) void k_sp24_bf16p(int nkt, const v4i
 // 16 bytes per row and pieces past kbytes, whose weights are the packing's
 // zeros, repeat the last one (the bf16 caller's XT is zero-padded to whole
 // steps instead, as 0 * inf is no zero).
+// XROW: the row-major activation itself (rows ldb bytes apart, 16-byte aligned,
+// N a multiple of a piece's 16 or 8 columns; pieces past N repeat the last
+// one), with kbytes = K: a step's k rows, 16 (bf16: 32) NB bytes of each, go to
+// LDS row by row (piece q of row r at q ^ 1 ((r >> 2) & 3), bf16 q ^ 2 ((r >> 1)
+// & 3), where NB = 4 would put rows of one read on the same banks) and the
+// fragments come from the transpose reads of k_sp24_i8 / k_sp24_bf16p.  Rows
+// past K repeat the last one (int8) or are zero (bf16).  It saves transposing
+// X first: int8 4096 x 4096 on 16 columns 8.0 -> 5.2 us, bf16 on 8 8.9 -> 5.7.
 // FLIP: x is uint8, taken as x - 128 (see k_sp24_i8).  Outputs: D's lane holds
 // rows 4 (l / 16) .. + 3 of column l % 16; with `trans` they go to Y[n][m]
 // (the x . W form, 16 bytes per lane), else to Y[m][n].
@@ -1094,7 +1102,7 @@ struct Sp24Epi {
     int out_kind, trans;
 };
 
-template <bool BF, int RB, int NB, int W, int D, bool FLIP>
+template <bool BF, int RB, int NB, int W, int D, bool FLIP, bool XROW>
 __global__ __launch_bounds__(64 * W) void k_sp24_small(int nsteps, int nkt, const v4i* __restrict__ A,
                                                        const uint32_t* __restrict__ I, const char* __restrict__ XT,
                                                        int64_t ldb, int kbytes, int M, int N, int ntn,
@@ -1117,18 +1125,26 @@ __global__ __launch_bounds__(64 * W) void k_sp24_small(int nsteps, int nkt, cons
     const int n0 = nt * 16 * NB;
     const v4i* aw[RB];
     const uint32_t* iw[RB];
-    const char* bw[2 * NB];  // rows 8h + l / 8 of the tile
 #pragma unroll
     for (int i = 0; i < RB; ++i) {
         aw[i] = A + (mb0 + i) * nkt * 64 + l;
         iw[i] = I + (mb0 + i) * (BF ? nkt / 2 : nkt) * 64 + l;
     }
+    // this lane's pieces of a step: XT: piece l % 8 of the tile's row 8h + l /
+    // 8; XROW: piece xq(h) of the step's k row xr(h)
+    constexpr int PR = BF ? 2 * NB : NB, KS = BF ? 64 : 128;  // pieces of an X row, k rows of a step
+    auto xr = [&](int h) { return (l + 64 * h) / PR; };
+    auto xq = [&](int h) { return (l + 64 * h) % PR; };
+    const char* bw[2 * NB];
 #pragma unroll
-    for (int h = 0; h < 2 * NB; ++h) bw[h] = XT + (int64_t)min(n0 + 8 * h + (l >> 3), N - 1) * ldb;
+    for (int h = 0; h < 2 * NB; ++h) {
+        if constexpr (XROW) bw[h] = XT + (BF ? 2 : 1) * min(n0 + (BF ? 8 : 16) * xq(h), N - (BF ? 8 : 16));
+        else bw[h] = XT + (int64_t)min(n0 + 8 * h + (l >> 3), N - 1) * ldb;
+    }
     char* const rows = lds + w * NB * 2048;
-    // this lane's piece of row 8h + l / 8: the swizzle (row >> 1) & 7 is (4h + l / 16) & 7
-    const int wr = (l >> 3) * 128, wp = l & 7;
+    const int wr = (l >> 3) * 128, wp = l & 7;  // the swizzle (row >> 1) & 7 of row 8h + l / 8 is (4h + l / 16) & 7
     const int rd = c * 128, rs = (c >> 1) & 7;
+    auto xswz = [](int r) { return NB < 4 ? 0 : (BF ? 2 * ((r >> 1) & 3) : (r >> 2) & 3); };
     struct Slot {
         v4i a[RB], b[2 * NB];
         uint32_t ix[RB];
@@ -1139,27 +1155,60 @@ __global__ __launch_bounds__(64 * W) void k_sp24_small(int nsteps, int nkt, cons
             f.a[i] = aw[i][(int64_t)s * 64];
             f.ix[i] = iw[i][(int64_t)(BF ? s >> 1 : s) * 64];
         }
-        const int o = min(128 * s + 16 * wp, kbytes - 16);
+        if constexpr (XROW) {
 #pragma unroll
-        for (int h = 0; h < 2 * NB; ++h) f.b[h] = *reinterpret_cast<const v4i*>(bw[h] + o);
+            for (int h = 0; h < 2 * NB; ++h)
+                f.b[h] = *reinterpret_cast<const v4i*>(bw[h] + (int64_t)min(KS * s + xr(h), kbytes - 1) * ldb);
+        } else {
+            const int o = min(128 * s + 16 * wp, kbytes - 16);
+#pragma unroll
+            for (int h = 0; h < 2 * NB; ++h) f.b[h] = *reinterpret_cast<const v4i*>(bw[h] + o);
+        }
         // keep this step's loads ahead of the MFMAs that follow
         __builtin_amdgcn_sched_barrier(0);
     };
     struct Frag {
         v8i b[NB];
     };
-    auto arrange = [&](Frag& g, const Slot& f) {
+    auto arrange = [&](Frag& g, const Slot& f, int s) {
 #pragma unroll
         for (int h = 0; h < 2 * NB; ++h) {
             v4i b = f.b[h];
             if constexpr (FLIP) b ^= (int)0x80808080;
-            *reinterpret_cast<v4i*>(rows + h * 1024 + wr + 16 * (wp ^ ((4 * h + (l >> 4)) & 7))) = b;
+            if constexpr (XROW) {
+                if constexpr (BF) {
+                    if (KS * (s + 1) > kbytes && KS * s + xr(h) >= kbytes) b = v4i{0, 0, 0, 0};
+                }
+                *reinterpret_cast<v4i*>(rows + xr(h) * (16 * PR) + 16 * (xq(h) ^ xswz(xr(h)))) = b;
+            } else {
+                *reinterpret_cast<v4i*>(rows + h * 1024 + wr + 16 * (wp ^ ((4 * h + (l >> 4)) & 7))) = b;
+            }
         }
 #pragma unroll
         for (int j = 0; j < NB; ++j) {
-            const v4i lo = *reinterpret_cast<const v4i*>(rows + j * 2048 + rd + 16 * (kb ^ rs));
-            const v4i hi = *reinterpret_cast<const v4i*>(rows + j * 2048 + rd + 16 * ((4 + kb) ^ rs));
-            g.b[j] = v8i{lo.x, lo.y, lo.z, lo.w, hi.x, hi.y, hi.z, hi.w};
+            if constexpr (XROW) {
+                // read r of this lane: row k0 + c / 2 (bf16: c / 4), its 8
+                // bytes c % 2 of the piece
+                typedef short v4s __attribute__((ext_vector_type(4)));
+                v2i q[4];
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    const int row = BF ? 8 * kb + 4 * (r & 1) + 32 * (r >> 1) + (c >> 2)
+                                       : 16 * kb + 8 * (r & 1) + 64 * (r >> 1) + (c >> 1);
+                    const int piece = BF ? 2 * j + ((c >> 1) & 1) : j;
+                    char* at = rows + row * (16 * PR) + 16 * (piece ^ xswz(row)) + 8 * (c & 1);
+                    if constexpr (BF)
+                        q[r] = __builtin_bit_cast(v2i, __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+                                                           (__attribute__((address_space(3))) v4s*)at));
+                    else
+                        q[r] = __builtin_amdgcn_ds_read_tr8_b64_v2i32((__attribute__((address_space(3))) v2i*)at);
+                }
+                g.b[j] = v8i{q[0].x, q[0].y, q[1].x, q[1].y, q[2].x, q[2].y, q[3].x, q[3].y};
+            } else {
+                const v4i lo = *reinterpret_cast<const v4i*>(rows + j * 2048 + rd + 16 * (kb ^ rs));
+                const v4i hi = *reinterpret_cast<const v4i*>(rows + j * 2048 + rd + 16 * ((4 + kb) ^ rs));
+                g.b[j] = v8i{lo.x, lo.y, lo.z, lo.w, hi.x, hi.y, hi.z, hi.w};
+            }
         }
         __builtin_amdgcn_sched_barrier(0);
     };
@@ -1191,23 +1240,23 @@ __global__ __launch_bounds__(64 * W) void k_sp24_small(int nsteps, int nkt, cons
 #pragma unroll
         for (int u = 0; u + 1 < D; ++u) load(r[u], step(u));
         constexpr bool AHEAD = D > 2;  // two slots: the other one has only just been asked for
-        if (AHEAD) arrange(g[0], r[0]);
+        if (AHEAD) arrange(g[0], r[0], step(0));
         int i = 0;
         static_assert(D % 2 == 0, "the fragment sets alternate");
         for (; i + D <= n; i += D) {
 #pragma unroll
             for (int u = 0; u < D; ++u) {
                 load(r[(u + D - 1) % D], step(i + u + D - 1));
-                if (AHEAD) arrange(g[(u + 1) % 2], r[(u + 1) % D]);  // (the last step's: once more)
-                else arrange(g[u % 2], r[u]);
+                if (AHEAD) arrange(g[(u + 1) % 2], r[(u + 1) % D], step(i + u + 1));  // (the last step's: once more)
+                else arrange(g[u % 2], r[u], step(i + u));
                 mma(r[u], g[u % 2], step(i + u));
             }
         }
 #pragma unroll
         for (int u = 0; u + 1 < D; ++u)
             if (i + u < n) {
-                if (!AHEAD) arrange(g[u % 2], r[u]);
-                else if (u + 2 < D) arrange(g[(u + 1) % 2], r[u + 1]);
+                if (!AHEAD) arrange(g[u % 2], r[u], step(i + u));
+                else if (u + 2 < D) arrange(g[(u + 1) % 2], r[u + 1], step(i + u + 1));
                 mma(r[u], g[u % 2], step(i + u));
             }
     }
@@ -1652,12 +1701,17 @@ constexpr SmallTile kSmallTiles[] = {{1, 1, 8, 3500, 870, 24},
                                      {4, 4, 4, 6000, 2000, 140}};
 
 // The tile (an index into kSmallTiles) that serves an M x N product of
-// `steps` 128-byte steps soonest, and its time in ns.
-int small_tile(const pfr_ctx* ctx, int64_t M, int64_t N, int64_t steps, int64_t* ns) {
+// `steps` 128-byte steps soonest, and its time in ns.  elem: 0 for XT, else
+// the element size of a row-major X read in place: then a tile narrower than
+// the rows reads pieces of lines (4096 x 4096 int8 on 128 columns: 64 x 32
+// tiles 13.0 us, against 7.3 after a transpose of 4), so only tiles as wide as
+// the rows, or the widest, are taken.
+int small_tile(const pfr_ctx* ctx, int64_t M, int64_t N, int64_t steps, int elem, int64_t* ns) {
     int best = 0;
     *ns = INT64_MAX;
     for (int i = 0; i < 5; ++i) {
         const SmallTile& t = kSmallTiles[i];
+        if (elem > 0 && t.nb < 4 && 16 * t.nb < N) continue;
         const int64_t wgs = (M + 16 * t.rb - 1) / (16 * t.rb) * ((N + 16 * t.nb - 1) / (16 * t.nb));
         const int64_t per_cu = (wgs + ctx->num_cu - 1) / ctx->num_cu;
         const int64_t e = t.start + per_cu * (t.each + steps * t.step);
@@ -1679,9 +1733,32 @@ int64_t large_ns(const pfr_ctx* ctx, const pfr_sp24* W, int64_t N, int64_t steps
 }
 constexpr int64_t kTransposeNs = 4000;
 
-// Launches the small-tile kernel: XT as it describes, Y and ep as set by the
-// caller.
-template <bool BF, bool FLIP>
+// How a W . X product runs: on the small tile `tile` (-1: the large ones),
+// reading X in place or its transpose.  pieces: X can be read in place by the
+// small tiles; xrow: by the large ones (the transpose, which takes scratch, is
+// then not considered).
+struct Plan24 {
+    int tile;
+    bool in_place;
+};
+Plan24 plan_small(const pfr_ctx* ctx, const pfr_sp24* W, int64_t N, int elem, bool pieces, bool xrow) {
+    const int64_t kstep = 128 / elem, steps = (W->K + kstep - 1) / kstep;
+    int64_t best = large_ns(ctx, W, N, W->Kp / kstep, xrow) + (xrow ? 0 : kTransposeNs), ns = 0;
+    Plan24 p{-1, false};
+    if (!xrow) {
+        const int t = small_tile(ctx, W->M, N, steps, 0, &ns);
+        if (ns + kTransposeNs < best) best = ns + kTransposeNs, p = {t, false};
+    }
+    if (pieces) {
+        const int t = small_tile(ctx, W->M, N, steps, elem, &ns);
+        if (ns < best) p = {t, true};
+    }
+    return p;
+}
+
+// Launches the small-tile kernel: XT, ldb and kbytes as it describes, Y and ep
+// as set by the caller.
+template <bool BF, bool FLIP, bool XROW>
 void launch_small(pfr_ctx* ctx, const pfr_sp24* W, int tile, const char* XT, int64_t ldb, int64_t kbytes, int64_t N,
                   void* Y, int64_t ldy, const Sp24Epi& ep) {
     const int nkt = (int)(W->Kp / (BF ? 64 : 128)), steps = (int)((W->K + (BF ? 63 : 127)) / (BF ? 64 : 128));
@@ -1690,7 +1767,7 @@ void launch_small(pfr_ctx* ctx, const pfr_sp24* W, int tile, const char* XT, int
         static_assert(kSmallTiles[IDX].rb == RBV && kSmallTiles[IDX].nb == NBV && kSmallTiles[IDX].w == WV, "tile"); \
         const int ntn = (int)((N + 16 * NBV - 1) / (16 * NBV));                                                     \
         const dim3 grid((unsigned)((W->M + 16 * RBV - 1) / (16 * RBV) * ntn));                                      \
-        hipLaunchKernelGGL((k_sp24_small<BF, RBV, NBV, WV, DV, FLIP>), grid, dim3(64 * WV), 0, ctx->stream, steps,  \
+        hipLaunchKernelGGL((k_sp24_small<BF, RBV, NBV, WV, DV, FLIP, XROW>), grid, dim3(64 * WV), 0, ctx->stream, steps,  \
                            nkt, static_cast<const v4i*>(W->a), W->idx, XT, ldb, (int)kbytes, (int)W->M, (int)N, ntn, \
                            Y, ldy, ep);                                                                             \
         break;                                                                                                      \
@@ -1743,19 +1820,27 @@ void gemm_i8_dev(pfr_ctx* ctx, const pfr_sp24* W, const int8_t* X, int64_t N, in
     // stay inside it and its rows are 16-byte aligned; otherwise it is
     // transposed into a zero-padded XT (Np x Kp) first.
     const bool xrow = W->K == Kp && N % kI8TileN == 0 && (x_u8 || aligned);
-    int64_t small_ns = 0;
-    const int tile = small_tile(ctx, W->M, N, (W->K + 127) / 128, &small_ns);
-    if (small_ns + (xrow ? kTransposeNs : 0) < large_ns(ctx, W, N, Kp / 128, xrow)) {
+    // the small tiles read X in place when its 16-byte pieces are whole, or
+    // its transpose; a call that the large tiles serve in place uses no
+    // scratch, and keeps it that way
+    const Plan24 plan = plan_small(ctx, W, N, 1, aligned && N % 16 == 0 && W->K > 0, xrow);
+    if (plan.tile >= 0) {
+        const Sp24Epi ep{W->w_scale, x_scale, inv_out, out_zp, inrange, x_zp, x_u8 ? 128 : 0, xs_dev, zp_dev,
+                         W->row_sum, out_kind, 0};
+        if (plan.in_place) {
+            const char* b = reinterpret_cast<const char*>(X);
+            if (x_u8) launch_small<false, true, true>(ctx, W, plan.tile, b, ldx, W->K, N, Y, ldy, ep);
+            else launch_small<false, false, true>(ctx, W, plan.tile, b, ldx, W->K, N, Y, ldy, ep);
+            return;
+        }
         const int64_t rows = round_up(N, 16);
-        int8_t* xt = static_cast<int8_t*>(ctx->scratch[3].ensure((size_t)(rows * Kp)));
+        int8_t* xt = static_cast<int8_t*>(ctx->scratch[3].ensure((size_t)(round_up(N, kI8TileN) * Kp)));
         hipLaunchKernelGGL(k_transpose_i8, dim3((unsigned)(Kp / 64), (unsigned)((rows + 255) / 256)), dim3(256), 0,
                            ctx->stream, X, W->K, N, ldx, aligned ? 1 : 0, xt, Kp, rows);
         PFR_HIP(hipGetLastError());
-        const Sp24Epi ep{W->w_scale, x_scale, inv_out, out_zp, inrange, x_zp, x_u8 ? 128 : 0, xs_dev, zp_dev,
-                         W->row_sum, out_kind, 0};
         const char* b = reinterpret_cast<const char*>(xt);
-        if (x_u8) launch_small<false, true>(ctx, W, tile, b, Kp, Kp, N, Y, ldy, ep);
-        else launch_small<false, false>(ctx, W, tile, b, Kp, Kp, N, Y, ldy, ep);
+        if (x_u8) launch_small<false, true, false>(ctx, W, plan.tile, b, Kp, Kp, N, Y, ldy, ep);
+        else launch_small<false, false, false>(ctx, W, plan.tile, b, Kp, Kp, N, Y, ldy, ep);
         return;
     }
     if (x_u8) {
@@ -1868,14 +1953,14 @@ void gemm_qt_dev(pfr_ctx* ctx, const pfr_sp24* W, const uint8_t* X, bool x_u8, i
     if (!xs_dev) pfr::require(x_scale > 0.0f && std::isfinite(x_scale), "x_scale must be positive and finite");
     const int64_t Kp = W->Kp, Np = round_up(T, kI8TileN), ldyp = round_up(T, 16);
     int64_t small_ns = 0;
-    const int tile = small_tile(ctx, W->M, T, (W->K + 127) / 128, &small_ns);
+    const int tile = small_tile(ctx, W->M, T, (W->K + 127) / 128, 0, &small_ns);
     if (small_ns < large_ns(ctx, W, T, Kp / 128, false) + 2 * kTransposeNs) {
         // the rows of X are the K-contiguous operand as they are, when their
         // 16-byte pieces are whole and aligned
         const bool direct = W->K >= 16 && W->K % 16 == 0 && ldx % 16 == 0 && (reinterpret_cast<uintptr_t>(X) & 15) == 0;
         const uint8_t* b = X;
         if (!direct) {
-            uint8_t* xt = static_cast<uint8_t*>(ctx->scratch[3].ensure((size_t)(T * Kp)));
+            uint8_t* xt = static_cast<uint8_t*>(ctx->scratch[3].ensure((size_t)(Np * Kp)));
             hipLaunchKernelGGL(k_pad_act<false>, dim3((unsigned)((T * Kp + 255) / 256)), dim3(256), 0, ctx->stream, X, T,
                                W->K, ldx, xt, Kp, T);
             PFR_HIP(hipGetLastError());
@@ -1884,8 +1969,8 @@ void gemm_qt_dev(pfr_ctx* ctx, const pfr_sp24* W, const uint8_t* X, bool x_u8, i
         const Sp24Epi ep{W->w_scale, x_scale, 1.0f, 0, 0, x_zp, x_u8 ? 128 : 0, xs_dev, zp_dev, W->row_sum,
                          PFR_SP24_OUT_F32, 1};
         const char* bc = reinterpret_cast<const char*>(b);
-        if (x_u8) launch_small<false, true>(ctx, W, tile, bc, direct ? ldx : Kp, direct ? W->K : Kp, T, Y, ldy, ep);
-        else launch_small<false, false>(ctx, W, tile, bc, direct ? ldx : Kp, direct ? W->K : Kp, T, Y, ldy, ep);
+        if (x_u8) launch_small<false, true, false>(ctx, W, tile, bc, direct ? ldx : Kp, direct ? W->K : Kp, T, Y, ldy, ep);
+        else launch_small<false, false, false>(ctx, W, tile, bc, direct ? ldx : Kp, direct ? W->K : Kp, T, Y, ldy, ep);
         return;
     }
     uint8_t* xt = static_cast<uint8_t*>(ctx->scratch[3].ensure((size_t)(Np * Kp)));
@@ -1919,17 +2004,22 @@ void gemm_bf16_dev(pfr_ctx* ctx, const pfr_sp24* W, const uint16_t* X, int64_t N
     // it is transposed into a zero-padded XT (Np x Kp) first.
     const bool xrow = W->K == W->Kp && N % kI8TileN == 0 && ldx % 8 == 0 &&
                       (reinterpret_cast<uintptr_t>(X) & 15) == 0;
-    int64_t small_ns = 0;
-    const int tile = small_tile(ctx, W->M, N, (W->K + 63) / 64, &small_ns);
+    const Plan24 plan = plan_small(ctx, W, N, 2, ldx % 8 == 0 && N % 8 == 0 && W->K > 0 &&
+                                                     (reinterpret_cast<uintptr_t>(X) & 15) == 0, xrow);
     const int vec = (ldx % 4 == 0 && (reinterpret_cast<uintptr_t>(X) & 7) == 0) ? 1 : 0;
-    if (small_ns + (xrow ? kTransposeNs : 0) < large_ns(ctx, W, N, W->Kp / 64, xrow)) {
-        const int64_t rows = round_up(N, 64);
-        uint16_t* xt = static_cast<uint16_t*>(ctx->scratch[3].ensure(sizeof(uint16_t) * (size_t)(rows * W->Kp)));
-        hipLaunchKernelGGL(k_transpose_b16, dim3((unsigned)(W->Kp / 64), (unsigned)(rows / 64)), dim3(256), 0,
+    if (plan.tile >= 0) {
+        if (plan.in_place) {
+            launch_small<true, false, true>(ctx, W, plan.tile, reinterpret_cast<const char*>(X), 2 * ldx, W->K, N, Y, ldy,
+                                            Sp24Epi{});
+            return;
+        }
+        uint16_t* xt = static_cast<uint16_t*>(
+            ctx->scratch[3].ensure(sizeof(uint16_t) * (size_t)(round_up(N, kI8TileN) * W->Kp)));
+        hipLaunchKernelGGL(k_transpose_b16, dim3((unsigned)(W->Kp / 64), (unsigned)(round_up(N, 64) / 64)), dim3(256), 0,
                            ctx->stream, X, W->K, N, ldx, vec, xt, W->Kp);
         PFR_HIP(hipGetLastError());
-        launch_small<true, false>(ctx, W, tile, reinterpret_cast<const char*>(xt), 2 * W->Kp, 2 * W->Kp, N, Y, ldy,
-                                  Sp24Epi{});
+        launch_small<true, false, false>(ctx, W, plan.tile, reinterpret_cast<const char*>(xt), 2 * W->Kp, 2 * W->Kp, N, Y, ldy,
+                                         Sp24Epi{});
         return;
     }
     const int64_t Np = round_up(N, kI8TileN);
