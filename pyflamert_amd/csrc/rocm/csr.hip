@@ -206,7 +206,7 @@ void sell_geom(int64_t K, int64_t* kc, int64_t* nch) {
 
 constexpr int kMaxCountChunks = 4096;  // sliced-ELL chunks counted in LDS by the device build (K <= 4M)
 
-// The sliced-ELL copy exists for float32 weights whose count table stays
+// The sliced-ELL copy exists for weights whose count table stays
 // small and whose chunks the device build can count in LDS (else the row
 // kernels serve), the same limit for the host and the device build, so
 // every product through either handle runs the same kernel.
@@ -759,11 +759,15 @@ __device__ __forceinline__ int32_t first_at_least(const CI* __restrict__ col, in
 // of chunk c is that chunk's step j - (the row's first entry in c); step t
 // of slab lane r in chunk c is int4 t / 8 * 64 + 4 r + t % 8 / 2 of the
 // (slab, chunk) run, its half t % 2.  blk holds the padding pattern.
-template <class CI>
+// An int8 weight's steps hold the float32 value its products use, RN((float)q *
+// row scale) (dequantize_tensor with zero point 0, quant_ops.cpp:182-196), so
+// the walk, and strict mode's bits, are those of that float32 weight.
+template <class CI, class V>
 __global__ __launch_bounds__(256) void k_sell_fill(int64_t npos, const int32_t* __restrict__ perm,
                                                    const int32_t* __restrict__ rowptr, const CI* __restrict__ col,
-                                                   const float* __restrict__ val, const int64_t* __restrict__ off,
-                                                   int nch, int kc, int4* __restrict__ blk) {
+                                                   const V* __restrict__ val, const float* __restrict__ rs,
+                                                   const int64_t* __restrict__ off, int nch, int kc,
+                                                   int4* __restrict__ blk) {
     const int64_t i = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
     if (i >= npos) return;
     const int lane = threadIdx.x & 63;
@@ -771,13 +775,14 @@ __global__ __launch_bounds__(256) void k_sell_fill(int64_t npos, const int32_t* 
     if (row < 0) return;  // a lane of a partial slab past its rows
     const int32_t b = rowptr[row], e = rowptr[row + 1];
     const int64_t sl = i / pfr::kSellRows, r = i % pfr::kSellRows;
+    const float scale = sizeof(V) == 1 ? rs[row] : 1.0f;
     for (int32_t j = b + lane; j < e; j += 64) {
         const int32_t k = (int32_t)col[j], c = k / kc;
         const int32_t step = j - first_at_least(col, b, j, c * kc);
         int32_t* q = reinterpret_cast<int32_t*>(blk + off[sl * nch + c] + (step / 8) * 64 + 4 * r + (step % 8) / 2) +
                      (step % 2) * 2;
         q[0] = (k - c * kc) * 64;
-        q[1] = __float_as_int(val[j]);
+        q[1] = __float_as_int(sizeof(V) == 1 ? (float)val[j] * scale : (float)val[j]);
     }
 }
 
@@ -1111,7 +1116,8 @@ void set_lazy(pfr_csr* w, const std::vector<int32_t>& rowptr, std::vector<int32_
               std::vector<int32_t> bal_cnt) {
     uint32_t bits = 0;
     if (w->M > 0 && w->nnz > 0) {
-        bits = pfr::kCopyChain | (sell_cnt.empty() ? 0u : pfr::kCopySell | pfr::kCopySellFast) |
+        const uint32_t sell = w->vdt == PFR_I8 ? pfr::kCopySell : pfr::kCopySell | pfr::kCopySellFast;
+        bits = pfr::kCopyChain | (sell_cnt.empty() ? 0u : sell) |
                (bal_cnt.empty() ? 0u : pfr::kCopyBal);
         w->h_rowptr = rowptr;
         w->h_sell_cnt = std::move(sell_cnt);
@@ -1126,8 +1132,9 @@ std::vector<int32_t> row_lengths(const pfr_csr* w) {
     return len;
 }
 
-// Sliced-ELL copy (float32 values), planned from the kept chunk counts.
-template <class CI>
+// Sliced-ELL copy (float32 steps, V the weight's values), planned from the
+// kept chunk counts.
+template <class CI, class V>
 void fill_sell(pfr_csr* w, const CI* col, hipStream_t s) {
     SellPlan p;
     if (!plan_sell(w->M, w->K, w->h_sell_cnt, &p)) return;
@@ -1137,8 +1144,8 @@ void fill_sell(pfr_csr* w, const CI* col, hipStream_t s) {
     if (w->sell_perm == nullptr) set_sell(w, p, s);  // else the fast copy's build uploaded them
     int64_t* off = dev_alloc_copy(p.off.data(), (int64_t)p.off.size(), s);
     const int64_t npos = p.nslab * pfr::kSellRows;  // perm's length
-    hipLaunchKernelGGL(k_sell_fill<CI>, dim3(waves_grid(npos)), dim3(256), 0, s, npos, w->sell_perm, w->rowptr, col,
-                       static_cast<const float*>(w->val), off, (int)p.nch, (int)p.kc, w->sell_blk);
+    hipLaunchKernelGGL((k_sell_fill<CI, V>), dim3(waves_grid(npos)), dim3(256), 0, s, npos, w->sell_perm, w->rowptr,
+                       col, static_cast<const V*>(w->val), w->row_scale, off, (int)p.nch, (int)p.kc, w->sell_blk);
     const hipError_t e = hipGetLastError();
     (void)hipStreamSynchronize(s);
     (void)hipFree(off);
@@ -1246,8 +1253,8 @@ void fill_bal(pfr_csr* w, const CI* col, hipStream_t s) {
 template <class CI>
 void build_copy(pfr_csr* w, uint32_t bit, const CI* col, hipStream_t s) {
     const bool i8 = w->vdt == PFR_I8;
-    if (bit == pfr::kCopySell) fill_sell(w, col, s);  // pending for float32 weights only
-    else if (bit == pfr::kCopySellFast) fill_sell_fast(w, col, s);  // likewise
+    if (bit == pfr::kCopySell) i8 ? fill_sell<CI, int8_t>(w, col, s) : fill_sell<CI, float>(w, col, s);
+    else if (bit == pfr::kCopySellFast) fill_sell_fast(w, col, s);  // pending for float32 weights only
     else if (bit == pfr::kCopyChain) i8 ? fill_chain<CI, int8_t>(w, col, s) : fill_chain<CI, float>(w, col, s);
     else i8 ? fill_bal<CI, int8_t>(w, col, s) : fill_bal<CI, float>(w, col, s);
 }
@@ -1336,7 +1343,7 @@ pfr_csr* build(pfr_ctx* ctx, int64_t M, int64_t K, const std::vector<int32_t>& r
         int64_t kc, nchs, nchb = 0, kcw = 1;
         sell_geom(K, &kc, &nchs);
         std::vector<int32_t> cs, cb;
-        if (vdt == PFR_F32 && sell_wanted(M, K, w->nnz) && chunks_ascend(rowptr, col, M, kc)) {
+        if (sell_wanted(M, K, w->nnz) && chunks_ascend(rowptr, col, M, kc)) {
             cs.assign((size_t)(M * nchs), 0);
             for (int64_t r = 0; r < M; ++r)
                 for (int32_t j = rowptr[r]; j < rowptr[r + 1]; ++j) ++cs[(size_t)(r * nchs + col[j] / kc)];

@@ -31,7 +31,11 @@ using pfr::bias_add;
 constexpr int kWaves = 4;  // waves per 256-thread workgroup
 constexpr int kSpmvThreads = 512;  // threads of the vector kernel's workgroup
 constexpr int kSpmvCap = 4096;     // products staged per workgroup chunk (16 KB)
-constexpr int64_t kSellMinN = 16;  // column-slice kernel from this many columns on
+// Column-slice kernel from this many columns on (below, the balanced and
+// row-chain kernels; on 12 columns its slice is a quarter empty and still
+// takes 18 us on the 4096 x 4096, 10 % weight, against 48 reading the CSR in
+// place, and 90 against 285 on the 30 % int8 one).
+constexpr int64_t kSellMinN = 9;
 
 // One 4-byte word per lane from base + off into LDS at dst + 4 lane, as a
 // buffer load (bytes: the buffer's size; a lane past it reads zero).  A
@@ -1597,34 +1601,40 @@ void launch_bal_fast8(pfr_ctx* ctx, const pfr_csr* W, const float* X, int N, int
                        W->row_scale, X, ldx, Y, ldy_r, ldy_c, bias, c_size, beta, act);
 }
 
-// At[k, i] = RN(alpha * A[i, k]) for A rows x cols (At cols x rows).
+// At[k, i] = RN(alpha * A[i, k]) for A rows x cols; At rows ld >= rows floats
+// apart.  One 64 x 64 tile per workgroup, every load issued before the first
+// LDS write (addresses clamped into the matrix).  (Guarded loads, one row
+// latency after the other, took 10.0 us on 99 x 5003.)
 __global__ __launch_bounds__(256) void k_transpose_scale(const float* __restrict__ A, int64_t rows,
                                                          int64_t cols, float alpha, int scale,
-                                                         float* __restrict__ At) {
+                                                         float* __restrict__ At, int64_t ld) {
     __shared__ float tile[64][65];
     const int tx = threadIdx.x & 63, ty = threadIdx.x >> 6;
     const int64_t c0 = (int64_t)blockIdx.x * 64, r0 = (int64_t)blockIdx.y * 64;
-    for (int i = ty; i < 64; i += 4) {
-        const int64_t r = r0 + i, c = c0 + tx;
-        if (r < rows && c < cols) {
-            const float v = A[r * cols + c];
-            tile[i][tx] = scale ? alpha * v : v;
-        }
+    const int64_t cc = c0 + tx < cols ? c0 + tx : cols - 1;
+    float v[16];
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+        const int64_t r = r0 + ty + 4 * i;
+        v[i] = A[(r < rows ? r : rows - 1) * cols + cc];
     }
+#pragma unroll
+    for (int i = 0; i < 16; ++i) tile[ty + 4 * i][tx] = scale ? alpha * v[i] : v[i];
     __syncthreads();
-    for (int i = ty; i < 64; i += 4) {
-        const int64_t c = c0 + i, r = r0 + tx;
-        if (c < cols && r < rows) At[c * rows + r] = tile[tx][i];
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+        const int64_t c = c0 + ty + 4 * i, r = r0 + tx;
+        if (c < cols && r < rows) At[c * ld + r] = tile[tx][ty + 4 * i];
     }
 }
 
-// The same transpose for rows and cols multiples of 4 and a 16-byte aligned
-// A: 16-byte loads and stores, every load issued before the first LDS
-// write (addresses clamped into the matrix, out-of-range values dropped).
-// Both LDS passes are free of bank conflicts (row pitch 65).
+// The same transpose for cols and ld multiples of 4 and a 16-byte aligned A:
+// 16-byte loads and stores (the last store of an At row may fill it up to ld
+// with repeats of A's last row).  Both LDS passes are free of bank conflicts
+// (row pitch 65).
 __global__ __launch_bounds__(256) void k_transpose_scale4(const float* __restrict__ A, int64_t rows,
                                                           int64_t cols, float alpha, int scale,
-                                                          float* __restrict__ At) {
+                                                          float* __restrict__ At, int64_t ld) {
     __shared__ float tile[64][65];
     const int t = threadIdx.x;
     const int64_t c0 = (int64_t)blockIdx.x * 64, r0 = (int64_t)blockIdx.y * 64;
@@ -1658,7 +1668,7 @@ __global__ __launch_bounds__(256) void k_transpose_scale4(const float* __restric
         const int lcol = (t >> 4) + 16 * i;
         const int64_t c = c0 + lcol, r = r0 + lr4;
         if (c < cols && r < rows)
-            *reinterpret_cast<float4*>(At + c * rows + r) =
+            *reinterpret_cast<float4*>(At + c * ld + r) =
                 make_float4(tile[lr4][lcol], tile[lr4 + 1][lcol], tile[lr4 + 2][lcol], tile[lr4 + 3][lcol]);
     }
 }
@@ -1910,7 +1920,7 @@ template <bool FAST, bool XVEC, int W, bool XT>
 __global__ __launch_bounds__((sell_threads<XVEC, W, XT>())) void k_spmm_sell(
     int N, int K, int kc, int nch, int nslab, const int32_t* __restrict__ perm,
     const int32_t* __restrict__ soff, const int4* __restrict__ blk, const float* __restrict__ X,
-    int64_t ldx, float* __restrict__ Y, int64_t ldy_r, int64_t ldy_c, int yvec,
+    int64_t ldx, int nx, float* __restrict__ Y, int64_t ldy_r, int64_t ldy_c, int yvec,
     const float* __restrict__ bias, int64_t c_size, float beta, int act, float alpha, int scale) {
     // two buffers of kc + 1 rows of 16 floats; row kc of each is zero
     extern __shared__ float4 xs[];
@@ -1929,10 +1939,11 @@ __global__ __launch_bounds__((sell_threads<XVEC, W, XT>())) void k_spmm_sell(
     // 4r+q copying row 16j+r, columns n0+4q .. n0+4q+3, to LDS bytes
     // j*1024 + 16*lane of the chunk's buffer.  Loads past the wave's share
     // repeat its last one, rows past K repeat the chunk's last row and
-    // columns past N repeat the last four; nothing reads those copies.
+    // columns past nx (N, or the readable columns of a padded X: a multiple
+    // of 4) repeat the last four; nothing uses those copies.
     const int nld = kc / 16;
     const int nd = (nld + W - 1) / W;
-    const float* xcol = X + min(n0 + q * 4, N - 4);
+    const float* xcol = X + min(n0 + q * 4, nx - 4);
     auto dma = [&](int c, int i) {
         const int j = min(wave + W * i, nld - 1);
         const int k0 = c * kc, last = min(kc, K - k0) - 1;
@@ -1940,23 +1951,18 @@ __global__ __launch_bounds__((sell_threads<XVEC, W, XT>())) void k_spmm_sell(
         lds_char* dst = (lds_char*)(xs + (c & 1) * bufq) + j * 1024;
         __builtin_amdgcn_global_load_lds(src, dst, 16, 0, 0);
     };
-    // Register staging (any N and alignment) of chunk c into its buffer.
-    auto stage_regs = [&](int c) {
-        const int k0 = c * kc, rows = min(kc, K - k0);
-        float4* xb = xs + (c & 1) * bufq;
-        for (int e = tid; e < kc * 4; e += NT) {
-            const int kr = e >> 2, n = n0 + (e & 3) * 4;
-            float4 v = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-            if (kr < rows) {
-                const float* xr = X + (int64_t)(k0 + kr) * ldx;
-                if (n < N) v.x = xr[n];
-                if (n + 1 < N) v.y = xr[n + 1];
-                if (n + 2 < N) v.z = xr[n + 2];
-                if (n + 3 < N) v.w = xr[n + 3];
-            }
-            xb[e] = v;
-        }
+    // The same for any N and alignment, a float per lane: load i copies rows
+    // 4j .. 4j + 3 of the chunk, lane l column l % 16 of row 4j + l / 16.
+    // (Staged through registers, each piece behind its bounds checks, N = 99
+    // on the 4096 x 4096, 10 % weight took 35.2 us strict.)
+    auto dma1 = [&](int c, int i) {
+        const int j = min(wave + W * i, kc / 4 - 1);
+        const int k0 = c * kc, last = min(kc, K - k0) - 1;
+        const float* src = X + min(n0 + (lane & 15), N - 1) + (int64_t)(k0 + min(j * 4 + (lane >> 4), last)) * ldx;
+        lds_char* dst = (lds_char*)(xs + (c & 1) * bufq) + j * 256;
+        __builtin_amdgcn_global_load_lds(src, dst, 4, 0, 0);
     };
+    const int nd1 = (kc / 4 + W - 1) / W;
     // XT staging of chunk c by threads t, t + nthr, ..: piece e is the float4
     // of A's row n0 + e % 16 at k = 4 (e / 16) (eight loads in flight,
     // clamped addresses), written as four floats of four LDS rows; piece e
@@ -1993,7 +1999,7 @@ __global__ __launch_bounds__((sell_threads<XVEC, W, XT>())) void k_spmm_sell(
         }
     };
     auto sync_chunk = [&]() {
-        if constexpr (XVEC && !XT) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // this wave's loads have landed
+        if constexpr (!XT) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // this wave's loads have landed
         __syncthreads();
     };
 
@@ -2046,7 +2052,7 @@ __global__ __launch_bounds__((sell_threads<XVEC, W, XT>())) void k_spmm_sell(
     } else if constexpr (XVEC) {
         for (int i = 0; i < nd; ++i) dma(0, i);
     } else {
-        stage_regs(0);
+        for (int i = 0; i < nd1; ++i) dma1(0, i);
     }
     sync_chunk();
     for (int c = 0; c < nch; ++c) {
@@ -2060,7 +2066,9 @@ __global__ __launch_bounds__((sell_threads<XVEC, W, XT>())) void k_spmm_sell(
             float4* nxt = xs + ((c + 1) & 1) * bufq;
             // the 16-wave launch (four waves per SIMD hide each other's
             // latencies) stages whole chunks between walks instead
-            if (XVEC && !XT && W <= 8 && more)
+            if constexpr (W == 4)
+                sell_walk_pipe<FAST>(blk, s0 + lane, T, xb, a0, a1, a2, a3);
+            else if (XVEC && !XT && W <= 8 && more)
                 sell_walk<FAST, true, DPI>(blk, s0 + lane, T, xb, nxt, xcol + (int64_t)k1 * ldx, ldx, lane, wave, W,
                                            nld - 1, min(kc, K - k1) - 1, d, a0, a1, a2, a3);
             else
@@ -2073,7 +2081,7 @@ __global__ __launch_bounds__((sell_threads<XVEC, W, XT>())) void k_spmm_sell(
             } else if constexpr (XVEC) {
                 for (; d < nd; ++d) dma(c + 1, d);
             } else {
-                stage_regs(c + 1);  // the other buffer: last read in chunk c - 1
+                for (int i = 0; i < nd1; ++i) dma1(c + 1, i);  // the other buffer: last read in chunk c - 1
             }
             sync_chunk();
         }
@@ -2125,7 +2133,7 @@ const int4* sell_runs(const pfr_csr* W, bool fast) {
 
 // Column-slice kernel launch with W waves per workgroup.
 template <bool FAST, bool XVEC, int W, bool XT>
-void launch_sell_w(pfr_ctx* ctx, const pfr_csr* Wt, const float* X, int N, int64_t ldx, float* Y,
+void launch_sell_w(pfr_ctx* ctx, const pfr_csr* Wt, const float* X, int N, int64_t ldx, int nx, float* Y,
                    int64_t ldy_r, int64_t ldy_c, int yvec, const float* bias, int64_t c_size, float beta, int act,
                    float alpha) {
     auto kern = k_spmm_sell<FAST, XVEC, W, XT>;
@@ -2141,7 +2149,7 @@ void launch_sell_w(pfr_ctx* ctx, const pfr_csr* Wt, const float* X, int N, int64
     dim3 grid((unsigned)((Wt->sell_nslab + W - 1) / W), (unsigned)((N + pfr::kSellCols - 1) / pfr::kSellCols));
     hipLaunchKernelGGL(kern, grid, dim3(sell_threads<XVEC, W, XT>()), lds, ctx->stream, N, (int)Wt->K,
                        Wt->sell_kc, Wt->sell_nch, Wt->sell_nslab, Wt->sell_perm, Wt->sell_soff, sell_runs(Wt, FAST), X, ldx,
-                       Y, ldy_r, ldy_c, yvec, bias, c_size, beta, act, alpha, alpha != 1.0f ? 1 : 0);
+                       nx, Y, ldy_r, ldy_c, yvec, bias, c_size, beta, act, alpha, alpha != 1.0f ? 1 : 0);
 }
 
 // Waves per workgroup of the column-slice launch for N columns, and its
@@ -2161,11 +2169,11 @@ int sell_waves(const pfr_ctx* ctx, const pfr_csr* Wt, int64_t N, int64_t* rounds
 }
 
 template <bool FAST, bool XVEC, bool XT>
-void launch_sell_x(pfr_ctx* ctx, const pfr_csr* Wt, const float* X, int N, int64_t ldx, float* Y,
+void launch_sell_x(pfr_ctx* ctx, const pfr_csr* Wt, const float* X, int N, int64_t ldx, int nx, float* Y,
                    int64_t ldy_r, int64_t ldy_c, int yvec, const float* bias, int64_t c_size, float beta, int act,
                    float alpha) {
 #define PFR_SELLW(WV) \
-    launch_sell_w<FAST, XVEC, WV, XT>(ctx, Wt, X, N, ldx, Y, ldy_r, ldy_c, yvec, bias, c_size, beta, act, alpha)
+    launch_sell_w<FAST, XVEC, WV, XT>(ctx, Wt, X, N, ldx, nx, Y, ldy_r, ldy_c, yvec, bias, c_size, beta, act, alpha)
     const int w = sell_waves(ctx, Wt, N);
     if (w == 16) PFR_SELLW(16);
     else if (w == 8) PFR_SELLW(8);
@@ -2174,13 +2182,15 @@ void launch_sell_x(pfr_ctx* ctx, const pfr_csr* Wt, const float* X, int N, int64
 }
 
 // xt: X is the transposed activation (see k_spmm_sell), alpha its scale.
-void launch_sell(pfr_ctx* ctx, const pfr_csr* Wt, const float* X, int N, int64_t ldx, float* Y,
+// padded: X's rows are readable up to round_up(N, 4) columns.
+void launch_sell(pfr_ctx* ctx, const pfr_csr* Wt, const float* X, int N, int64_t ldx, bool padded, float* Y,
                  int64_t ldy_r, int64_t ldy_c, const float* bias, int64_t c_size, float beta, bool fast, int act,
                  bool xt = false, float alpha = 1.0f) {
-    const bool xvec = (ldx % 4 == 0) && (N % 4 == 0) && aligned16(X);
+    const int nx = padded ? (N + 3) / 4 * 4 : N;
+    const bool xvec = (ldx % 4 == 0) && (nx % 4 == 0) && aligned16(X);
     const int yvec = (ldy_c == 1 && ldy_r % 4 == 0 && aligned16(Y) && bias == nullptr) ? 1 : 0;
 #define PFR_SELLX(F, XV, T) \
-    launch_sell_x<F, XV, T>(ctx, Wt, X, N, ldx, Y, ldy_r, ldy_c, yvec, bias, c_size, beta, act, alpha)
+    launch_sell_x<F, XV, T>(ctx, Wt, X, N, ldx, nx, Y, ldy_r, ldy_c, yvec, bias, c_size, beta, act, alpha)
     if (xt) {
         if (fast) PFR_SELLX(true, false, true);
         else PFR_SELLX(false, false, true);
@@ -2355,11 +2365,11 @@ __global__ __launch_bounds__(256) void k_nonfinite_fix(const float* __restrict__
     }
 }
 
-// The column-slice kernel serves this product (float32 weight, N >= 16):
-// the fast mode runs on either sliced-ELL copy (its own when built), the
-// strict mode on the storage-order one.
+// The column-slice kernel serves this product (N >= kSellMinN): the fast mode
+// runs on either sliced-ELL copy (its own when built), the strict mode on the
+// storage-order one.
 bool sell_serves(const pfr_csr* W, int64_t N, bool fast) {
-    return W->vdt != PFR_I8 && N >= kSellMinN && sell_runs(W, fast) != nullptr &&
+    return N >= kSellMinN && sell_runs(W, fast) != nullptr &&
            N < (int64_t)pfr::kSellCols * 65535;
 }
 
@@ -2374,15 +2384,16 @@ bool sell_one_round(const pfr_ctx* ctx, const pfr_csr* W, int64_t N) {
 
 // Launch the kernel that fits N.  Output (row, c) -> Y[row*ldy_r + c*ldy_c].
 // xt: X is the Gemm form's activation A (N x K, rows ldx apart) read in
-// place, scaled by alpha; only where sell_serves.
+// place, scaled by alpha; only where sell_serves.  padded: X's rows are
+// readable up to round_up(N, 4) columns.
 void launch_spmm(pfr_ctx* ctx, const pfr_csr* W, const float* X, int64_t N, int64_t ldx, float* Y,
                  int64_t ldy_r, int64_t ldy_c, const float* bias, int64_t c_size, float beta,
-                 bool fast, int act, bool xt = false, float alpha = 1.0f) {
+                 bool fast, int act, bool padded = false, bool xt = false, float alpha = 1.0f) {
     if (W->M == 0 || N == 0) return;
     const bool i8 = W->vdt == PFR_I8;
     pfr::require(!xt || sell_serves(W, N, fast), "transposed activation without the column-slice copy");
     if (sell_serves(W, N, fast)) {
-        launch_sell(ctx, W, X, (int)N, ldx, Y, ldy_r, ldy_c, bias, c_size, beta, fast, act, xt, alpha);
+        launch_sell(ctx, W, X, (int)N, ldx, padded, Y, ldy_r, ldy_c, bias, c_size, beta, fast, act, xt, alpha);
     } else if (i8) {
         if (fast) launch_csr_kernels<true, true>(ctx, W, X, N, ldx, Y, ldy_r, ldy_c, bias, c_size, beta, act);
         else launch_csr_kernels<false, true>(ctx, W, X, N, ldx, Y, ldy_r, ldy_c, bias, c_size, beta, act);
@@ -2415,7 +2426,8 @@ void check_act(int act) {
 // when the handle still has it pending (its first such product).
 void ensure_copies(const pfr_ctx* ctx, const pfr_csr* W, int64_t N, bool fast) {
     uint32_t need = 0;
-    if (W->vdt == PFR_F32 && N >= kSellMinN) need |= fast ? pfr::kCopySellFast : pfr::kCopySell;
+    // (an int8 weight has the storage-order copy only, for both modes)
+    if (N >= kSellMinN) need |= fast && W->vdt != PFR_I8 ? pfr::kCopySellFast : pfr::kCopySell;
     if (fast && ((N >= 2 && N <= 8) || (N == 1 && !(ctx->merge && W->mp_wave != nullptr)))) need |= pfr::kCopyBal;
     if (!fast && N <= 8) need |= pfr::kCopyChain;
     if ((W->pending.load(std::memory_order_acquire) & need) != 0) pfr::csr_build_copies(const_cast<pfr_csr*>(W), need);
@@ -2452,11 +2464,16 @@ void gemm_dev(pfr_ctx* ctx, const float* A, int64_t Mb, int64_t K, int transA, c
         C = nullptr;
         c_size = 0;
     }
-    // At = op(A)^T scaled by alpha: K x Mb, so each k row is contiguous.
+    // At = op(A)^T scaled by alpha: K x Mb, so each k row is contiguous.  A
+    // transposed copy has its rows padded to whole 16-byte pieces (the
+    // allocation-free entry's workspace holds K * Mb as it is).
     const float* At = A;
+    int64_t ldt = Mb;
+    const bool pad = ws == nullptr && !transA && Mb >= kSellMinN;
+    if (pad) ldt = (Mb + 3) / 4 * 4;
     hipStream_t s = ctx->stream;
     auto tbuf = [&]() -> float* {
-        if (ws == nullptr) return static_cast<float*>(ctx->scratch[3].ensure(sizeof(float) * (size_t)(K * Mb)));
+        if (ws == nullptr) return static_cast<float*>(ctx->scratch[3].ensure(sizeof(float) * (size_t)(K * ldt)));
         pfr::require(K * Mb <= ws_floats,
                      "allocation-free Gemm: op(A) has K * Mb = " + std::to_string(K * Mb) +
                          " elements, more than its workspace of " + std::to_string(ws_floats) + " floats");
@@ -2464,6 +2481,8 @@ void gemm_dev(pfr_ctx* ctx, const float* A, int64_t Mb, int64_t K, int transA, c
     };
     if (K == 0) {
         // No terms: every output is +0 (+ bias); At is never read.
+    } else if (Mb == 1 && alpha == 1.0f) {
+        // one row: A is its own transpose
     } else if (!transA && ws == nullptr && sell_serves(BT, Mb, mode == PFR_MODE_FAST) && K % 4 == 0 && aligned16(A) &&
                sell_one_round(ctx, BT, Mb)) {
         // the column-slice kernel stages A's rows itself, transposed and
@@ -2473,18 +2492,18 @@ void gemm_dev(pfr_ctx* ctx, const float* A, int64_t Mb, int64_t K, int transA, c
         // a transposed A, so this pays off when the launch runs in one round
         // (every workgroup stages once, side by side): 768 x 768 at 1024
         // tokens 26.0 -> 21.7 us; 3072 x 768 (three rounds) 66.1 -> 67.8 us.
-        launch_spmm(ctx, BT, A, Mb, K, Y, 1, Nf, C, c_size, beta, mode == PFR_MODE_FAST, act, true, alpha);
+        launch_spmm(ctx, BT, A, Mb, K, Y, 1, Nf, C, c_size, beta, mode == PFR_MODE_FAST, act, false, true, alpha);
         return;
     } else if (!transA) {
         float* t = tbuf();
         dim3 grid((unsigned)((K + 63) / 64), (unsigned)((Mb + 63) / 64));
         pfr::require(grid.y < 65536u, "activation too tall for the transpose grid");
-        if (Mb % 4 == 0 && K % 4 == 0 && (reinterpret_cast<uintptr_t>(A) & 15) == 0)
+        if (ldt % 4 == 0 && K % 4 == 0 && (reinterpret_cast<uintptr_t>(A) & 15) == 0)
             hipLaunchKernelGGL(k_transpose_scale4, grid, dim3(256), 0, s, A, Mb, K, alpha,
-                               alpha != 1.0f ? 1 : 0, t);
+                               alpha != 1.0f ? 1 : 0, t, ldt);
         else
             hipLaunchKernelGGL(k_transpose_scale, grid, dim3(256), 0, s, A, Mb, K, alpha,
-                               alpha != 1.0f ? 1 : 0, t);
+                               alpha != 1.0f ? 1 : 0, t, ldt);
         PFR_HIP(hipGetLastError());
         At = t;
     } else if (alpha != 1.0f) {
@@ -2496,7 +2515,7 @@ void gemm_dev(pfr_ctx* ctx, const float* A, int64_t Mb, int64_t K, int transA, c
     }
     // Output (feature j, batch i) -> Y[i * Nf + j]: the flat index the bias
     // modulo uses in cpu_gemm.
-    launch_spmm(ctx, BT, At, Mb, Mb, Y, 1, Nf, C, c_size, beta, mode == PFR_MODE_FAST, act);
+    launch_spmm(ctx, BT, At, Mb, ldt, Y, 1, Nf, C, c_size, beta, mode == PFR_MODE_FAST, act, pad);
 }
 
 std::mutex g_ws_mu;
