@@ -113,6 +113,10 @@ struct DevBuf {
 
 }  // namespace pfr
 
+namespace pfr {
+constexpr size_t kPinnedBytes = size_t(1) << 20;
+}
+
 struct pfr_ctx {
     int device = 0;
     int num_cu = 256;
@@ -126,12 +130,21 @@ struct pfr_ctx {
     // transposed activations of the Gemm form, scratch[4]: the magnitude
     // mask's selection state (histogram, counters, per-block tie counts).
     // scratch[5]: the product before its transpose in the 2:4 x . W form.
-    pfr::DevBuf scratch[6];
+    // scratch[6]: the row and chunk counts of a CSR built on the device.
+    pfr::DevBuf scratch[7];
+    // Page-locked host memory (pfr::kPinnedBytes, allocated on first use) that
+    // weight builds send their small tables through; build_mu guards it and
+    // scratch[6] (a build that finds them taken uses memory of its own).
+    void* pinned = nullptr;
+    std::mutex build_mu;
 };
 
 struct pfr_csr {
     pfr_ctx* ctx = nullptr;
     int64_t M = 0, K = 0, nnz = 0;
+    // One allocation holding the arrays a build makes: rowptr, the columns,
+    // val, row_scale, spmv_blocks and the merge-path tables.
+    void* base = nullptr;
     int32_t* rowptr = nullptr;  // [M+1]
     // The columns in storage order, in one of two widths: col16 when K <=
     // 65536 (col is then null), else col.  col16 and val are padded to whole
@@ -148,7 +161,8 @@ struct pfr_csr {
     int32_t max_row_nnz = 0;
     // Columns ascend within every row (the order to_sparse produces).
     bool cols_sorted = false;
-    // Sliced-ELL copy of a float32 weight for the column-slice kernel (null
+    // Sliced-ELL copy for the column-slice kernel (float32 steps, also for int8
+    // values; null
     // when the shape does not qualify).  Rows are reordered into slabs of
     // kSellRows; K is cut into chunks of sell_kc rows (a multiple of 16, at
     // most kSellMaxKC; the last chunk may be partial).  For slab s and chunk
@@ -159,7 +173,7 @@ struct pfr_csr {
     // run is a multiple of kSellStepPad steps; padding steps point at the
     // zero row (offset sell_kc * 64, value +0).
     int32_t* sell_perm = nullptr;  // [sell_nslab * kSellRows] row of each slab lane, -1 none
-    int32_t* sell_soff = nullptr;  // [sell_nslab * (sell_nch + 1)]
+    int32_t* sell_soff = nullptr;  // [sell_nslab * (sell_nch + 1)], in sell_perm's allocation
     int4* sell_blk = nullptr;      // [sell_len + kSellTail]
     // The same runs for the fast mode (reassociated sums), each row's steps
     // of a chunk reordered so that at every step the four slab rows whose

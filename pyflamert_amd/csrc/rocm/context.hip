@@ -70,6 +70,7 @@ int pfr_rocm_destroy(pfr_ctx* ctx) {
         pfr::bind(ctx);
         (void)hipStreamSynchronize(ctx->stream);
         for (auto& b : ctx->scratch) b.release();
+        if (ctx->pinned) (void)hipHostFree(ctx->pinned);
         if (ctx->own_stream) (void)hipStreamDestroy(ctx->own_stream);
         delete ctx;
     });

@@ -70,15 +70,78 @@ T* walloc_copy(pfr_csr* w, const T* host, int64_t count, hipStream_t s) {
 
 void free_csr(pfr_csr* w) {
     if (!w) return;
-    for (void* p : {(void*)w->rowptr, (void*)w->col, w->val, (void*)w->row_scale, (void*)w->spmv_blocks,
-                    (void*)w->sell_perm, (void*)w->sell_soff, (void*)w->sell_blk, (void*)w->sell_blk_fast,
-                    (void*)w->chain_q0, (void*)w->col16,
-                    (void*)w->chain_len, (void*)w->chain_perm, w->chain_val, w->chain_col, (void*)w->bal_meta,
-                    (void*)w->bal_cmeta, (void*)w->bal_perm, (void*)w->bal_pair, w->bal_val, (void*)w->bal_col, (void*)w->pattern,
-                    (void*)w->mp_wave, (void*)w->mp_wmeta, (void*)w->mp_grp, (void*)w->mp_xchg,
-                    (void*)w->mp_carry, (void*)w->mp_cnt})
+    for (void* p : {w->base, (void*)w->sell_perm, (void*)w->sell_blk, (void*)w->sell_blk_fast,
+                    (void*)w->chain_q0, (void*)w->chain_len, (void*)w->chain_perm, w->chain_val, w->chain_col,
+                    (void*)w->bal_meta, (void*)w->bal_cmeta, (void*)w->bal_perm, (void*)w->bal_pair, w->bal_val,
+                    (void*)w->bal_col, (void*)w->pattern})
         if (p) (void)hipFree(p);
     delete w;
+}
+
+// Host bytes on their way to or from the device: the context's pinned buffer
+// where they fit and no other build is using it (a pageable copy of a few KB
+// costs about 50 us of host time, a pinned one about 10), else memory of its
+// own.  Its copies must have completed before it goes out of scope.
+struct Staging {
+    char* p = nullptr;
+    std::unique_lock<std::mutex> lock;  // held: this build owns the context's build buffers
+    std::vector<char> own;
+    Staging() = default;
+    Staging(pfr_ctx* ctx, size_t bytes) : lock(ctx->build_mu, std::try_to_lock) {
+        if (lock.owns_lock() && bytes <= pfr::kPinnedBytes) {
+            if (ctx->pinned == nullptr && hipHostMalloc(&ctx->pinned, pfr::kPinnedBytes, hipHostMallocDefault) != hipSuccess) {
+                (void)hipGetLastError();
+                ctx->pinned = nullptr;
+            }
+            p = static_cast<char*>(ctx->pinned);
+        }
+        if (p == nullptr) {
+            own.resize(bytes > 0 ? bytes : 1);
+            p = own.data();
+        }
+    }
+};
+
+// Stable sort of b[0, n) by key(b[i]), largest first: by counting where the
+// keys' range is not much larger than n, which is the plans' usual case (row
+// and chunk counts; std::stable_sort made up most of a 4096-row sliced-ELL
+// plan).
+template <class Key>
+void sort_desc(int32_t* b, int64_t n, Key key) {
+    if (n < 2) return;
+    int32_t lo = INT32_MAX, hi = INT32_MIN;
+    thread_local std::vector<int32_t> k, at, out;
+    k.resize((size_t)n);
+    for (int64_t i = 0; i < n; ++i) {
+        k[(size_t)i] = key(b[i]);
+        lo = std::min(lo, k[(size_t)i]);
+        hi = std::max(hi, k[(size_t)i]);
+    }
+    if (lo == hi) return;
+    out.resize((size_t)n);
+    if (n <= 64) {  // insertion
+        for (int64_t i = 1; i < n; ++i) {
+            const int32_t kv = k[(size_t)i], v = b[i];
+            int64_t j = i;
+            for (; j > 0 && k[(size_t)j - 1] < kv; --j) {
+                k[(size_t)j] = k[(size_t)j - 1];
+                b[j] = b[j - 1];
+            }
+            k[(size_t)j] = kv;
+            b[j] = v;
+        }
+        return;
+    }
+    const int64_t range = (int64_t)hi - lo + 1;
+    if (range > 8 * n) {
+        std::stable_sort(b, b + n, [&](int32_t x, int32_t y) { return key(x) > key(y); });
+        return;
+    }
+    at.assign((size_t)range + 1, 0);
+    for (int64_t i = 0; i < n; ++i) ++at[(size_t)(hi - k[(size_t)i]) + 1];
+    for (int64_t r = 0; r < range; ++r) at[(size_t)r + 1] += at[(size_t)r];
+    for (int64_t i = 0; i < n; ++i) out[(size_t)at[(size_t)(hi - k[(size_t)i])]++] = b[i];
+    std::copy(out.begin(), out.begin() + n, b);
 }
 
 // Greedy row blocks of <= kSpmvBudget nnz and <= kSpmvMaxRows rows; a longer
@@ -113,9 +176,7 @@ void sell_order(const std::vector<int32_t>& cnt, int64_t nch, int32_t* b, int64_
     const int64_t R = pfr::kSellRows;
     if (n <= R) return;
     const int64_t c = depth % nch;
-    std::stable_sort(b, b + n, [&](int32_t x, int32_t y) {
-        return cnt[(size_t)(x * nch + c)] > cnt[(size_t)(y * nch + c)];
-    });
+    sort_desc(b, n, [&](int32_t x) { return cnt[(size_t)(x * nch + c)]; });
     const int64_t h = (n / 2 + R - 1) / R * R;  // R <= h < n for n > R
     sell_order(cnt, nch, b, h, depth + 1);
     sell_order(cnt, nch, b + h, n - h, depth + 1);
@@ -253,27 +314,31 @@ bool plan_sell(int64_t M, int64_t K, const std::vector<int32_t>& cnt, SellPlan* 
     return p->len + pfr::kSellTail <= INT32_MAX;
 }
 
-// Uploads the plan's tables (sell_blk is set by the fill).
-void set_sell(pfr_csr* w, const SellPlan& p, hipStream_t s) {
-    std::vector<int32_t> soff((size_t)(p.nslab * (p.nch + 1)));
+// Uploads the plan's tables (sell_blk is set by the fill): one allocation, the
+// row order and then the run offsets.
+void set_sell(pfr_csr* w, const SellPlan& p, Staging& st, hipStream_t s) {
+    const int64_t np = (int64_t)p.perm.size(), ns = p.nslab * (p.nch + 1);
+    w->sell_perm = walloc<int32_t>(w, np + ns);
+    w->sell_soff = w->sell_perm + np;
+    auto* h = reinterpret_cast<int32_t*>(st.p);
+    std::copy(p.perm.begin(), p.perm.end(), h);
     for (int64_t sl = 0; sl < p.nslab; ++sl)
         for (int64_t c = 0; c <= p.nch; ++c)  // c == nch: end of the slab's last run
-            soff[(size_t)(sl * (p.nch + 1) + c)] = (int32_t)p.off[(size_t)(sl * p.nch + c)];
-    w->sell_perm = walloc_copy(w, p.perm.data(), (int64_t)p.perm.size(), s);
-    w->sell_soff = walloc_copy(w, soff.data(), (int64_t)soff.size(), s);
+            h[np + sl * (p.nch + 1) + c] = (int32_t)p.off[(size_t)(sl * p.nch + c)];
+    PFR_HIP(hipMemcpyAsync(w->sell_perm, h, sizeof(int32_t) * (size_t)(np + ns), hipMemcpyHostToDevice, s));
     w->sell_nslab = (int32_t)p.nslab;
     w->sell_nch = (int32_t)p.nch;
     w->sell_kc = (int32_t)p.kc;
     w->sell_len = p.len;
-    PFR_HIP(hipStreamSynchronize(s));  // soff goes out of scope
 }
+size_t sell_table_bytes(const SellPlan& p) { return sizeof(int32_t) * (p.perm.size() + (size_t)(p.nslab * (p.nch + 1))); }
 
 // Rows sorted by count, longest first, ties by row index (the row order of
 // the row-chain and balanced copies).
 std::vector<int32_t> order_by_length(const std::vector<int32_t>& len) {
     std::vector<int32_t> order(len.size());
     std::iota(order.begin(), order.end(), 0);
-    std::stable_sort(order.begin(), order.end(), [&](int32_t a, int32_t b) { return len[a] > len[b]; });
+    sort_desc(order.data(), (int64_t)order.size(), [&](int32_t a) { return len[(size_t)a]; });
     return order;
 }
 
@@ -480,15 +545,24 @@ void set_bal(pfr_csr* w, const BalPlan& p, hipStream_t s) {
 // workgroup's load stays within a row of C (on the int8 decode weights at
 // 30 % with lognormal rows the heaviest holds 1.007 to 1.041 times the
 // mean).  Within a workgroup the waves take shares weighted by their issue
-// priority (below).  Uploads
-// the tables and zeroes the exchange words and arrival counters.  False (no
-// partition) when the weight has no column copy in uint16 or x does not fit
-// the staged slot.
-bool set_merge(pfr_csr* w, const std::vector<int32_t>& rowptr, hipStream_t s) {
-    const int64_t M = w->M, nnz = w->nnz, T = M + nnz, W = pfr::kMergeWaves;
-    if (w->col16 == nullptr || nnz == 0 || w->K > pfr::kMergeMaxK || nnz > INT32_MAX - 4096) return false;
+// priority (below).  There is no partition (merge_wanted) when the weight has
+// no column copy in uint16 or x does not fit the staged slot.
+struct MergePlan {
+    int64_t P = 0;  // workgroups (0: no partition)
+    std::vector<int2> wave;
+    std::vector<int4> wmeta, grp;
+};
+// Most workgroups a partition may have.
+int64_t merge_groups_bound(const pfr_csr* w) {
     const int64_t cu = w->ctx->num_cu > 0 ? w->ctx->num_cu : 256;
-    const int64_t P0 = std::max<int64_t>(1, std::min<int64_t>(cu, T / (W * pfr::kMergeMinItems)));
+    return std::max<int64_t>(1, std::min<int64_t>(cu, (w->M + w->nnz) / (pfr::kMergeWaves * pfr::kMergeMinItems)));
+}
+bool merge_wanted(const pfr_csr* w) {
+    return w->K <= 65536 && w->nnz > 0 && w->K <= pfr::kMergeMaxK && w->nnz <= INT32_MAX - 4096;
+}
+MergePlan plan_merge(const pfr_csr* w, const int32_t* rowptr) {
+    const int64_t M = w->M, nnz = w->nnz, T = M + nnz, W = pfr::kMergeWaves;
+    const int64_t P0 = merge_groups_bound(w);
     std::vector<int64_t> ends((size_t)M);  // the diagonal just after row r's end
     for (int64_t r = 0; r < M; ++r) ends[(size_t)r] = rowptr[(size_t)r + 1] + r + 1;
     auto greedy = [&](int64_t C, std::vector<int64_t>* D) {
@@ -503,7 +577,9 @@ bool set_merge(pfr_csr* w, const std::vector<int32_t>& rowptr, hipStream_t s) {
         }
         return n;
     };
-    int64_t lo = (T + P0 - 1) / P0, hi = T;
+    // (a capacity of a mean share and the longest row is always enough: every
+    // workgroup but the last then takes at least a mean share)
+    int64_t lo = (T + P0 - 1) / P0, hi = std::min<int64_t>(T, lo + w->max_row_nnz + 1);
     while (lo < hi) {
         const int64_t mid = lo + (hi - lo) / 2;
         if (greedy(mid, nullptr) <= P0) hi = mid;
@@ -511,8 +587,9 @@ bool set_merge(pfr_csr* w, const std::vector<int32_t>& rowptr, hipStream_t s) {
     }
     std::vector<int64_t> D;
     const int64_t P = greedy(lo, &D);
-    auto search = [&](int64_t d) {
-        int64_t i0 = std::max<int64_t>(d - nnz, 0), i1 = std::min<int64_t>(d, M);
+    // (from row r0 to row r1, between which the coordinate is known to lie)
+    auto search = [&](int64_t d, int64_t r0, int64_t r1) {
+        int64_t i0 = std::max<int64_t>(d - nnz, r0), i1 = std::min<int64_t>(d, r1);
         while (i0 < i1) {
             const int64_t mid = i0 + (i1 - i0) / 2;
             if (rowptr[(size_t)mid + 1] <= d - mid - 1) i0 = mid + 1;
@@ -524,7 +601,7 @@ bool set_merge(pfr_csr* w, const std::vector<int32_t>& rowptr, hipStream_t s) {
     // nonzeros): the point of the path at that nonzero where every row
     // ending before it has ended, and a row ending exactly there keeps the
     // side the diagonal gave it
-    const auto e1 = rowptr.begin() + 1;
+    const int32_t* const e1 = rowptr + 1;
     const int64_t Q = P * W;
     // Wave t's share is proportional to kMergeWaveWeight[t].  The 16 waves
     // of a workgroup run four to a SIMD, and the SIMD's issue arbitration
@@ -543,14 +620,17 @@ bool set_merge(pfr_csr* w, const std::vector<int32_t>& rowptr, hipStream_t s) {
     }
     std::vector<int2> wp((size_t)Q + 1);
     for (int64_t p = 0; p < P; ++p) {
-        const int2 end = search(D[(size_t)p + 1]);
-        wp[(size_t)(p * W)] = search(D[(size_t)p]);
+        const int2 begin = search(D[(size_t)p], 0, M), end = search(D[(size_t)p + 1], begin.x, M);
+        wp[(size_t)(p * W)] = begin;
         for (int64_t t = 1; t < W; ++t) {
-            const int2 c = search(D[(size_t)p] + (int64_t)((double)(D[(size_t)p + 1] - D[(size_t)p]) * cum[t] / cum[W]));
+            const int2 c = search(D[(size_t)p] + (int64_t)((double)(D[(size_t)p + 1] - D[(size_t)p]) * cum[t] / cum[W]),
+                                  begin.x, end.x);
             const int2 prev = wp[(size_t)(p * W + t - 1)];
             const int64_t j = std::max<int64_t>(std::min<int64_t>(((int64_t)c.y + 3) / 4 * 4, end.y), prev.y);
-            const int64_t lt = std::lower_bound(e1, e1 + M, (int32_t)j) - e1;  // rows ending before j
-            const int64_t le = std::upper_bound(e1, e1 + M, (int32_t)j) - e1;  // rows ending at or before j
+            // rows ending before j and at or before j, among the workgroup's
+            // (any others would not change i)
+            const int64_t lt = std::lower_bound(e1 + begin.x, e1 + end.x, (int32_t)j) - e1;
+            const int64_t le = std::upper_bound(e1 + begin.x, e1 + end.x, (int32_t)j) - e1;
             const int64_t i = std::max<int64_t>(std::min<int64_t>(std::max<int64_t>(c.x, lt), le), prev.x);
             wp[(size_t)(p * W + t)] = make_int2((int)i, (int)j);
         }
@@ -614,17 +694,85 @@ bool set_merge(pfr_csr* w, const std::vector<int32_t>& rowptr, hipStream_t s) {
             wm[(size_t)(p * W + t)] = m;
         }
     }
-    w->mp_wave = walloc_copy(w, wp.data(), Q + 1, s);
-    w->mp_wmeta = walloc_copy(w, wm.data(), Q, s);
-    w->mp_grp = walloc_copy(w, gp.data(), P, s);
-    w->mp_xchg = walloc<unsigned long long>(w, P);
-    fill_dev(w->mp_xchg, P, 0ull, s);
-    w->mp_carry = walloc<float>(w, 2 * P);
-    w->mp_cnt = walloc<uint32_t>(w, P);
-    fill_dev(w->mp_cnt, P, 0u, s);
-    w->mp_groups = (int32_t)P;
-    PFR_HIP(hipStreamSynchronize(s));  // wp and gp outlive the uploads
-    return true;
+    MergePlan plan;
+    plan.P = P;
+    plan.wave = std::move(wp);
+    plan.wmeta = std::move(wm);
+    plan.grp = std::move(gp);
+    return plan;
+}
+
+// The handle's base arrays, carved from one allocation: the small tables
+// first, laid out alike on the host and the device so that they go over in
+// one or two copies (row pointers; then row scales, row blocks and the
+// merge-path tables with their zeroed exchange words and counters), then the
+// columns and the values.  (One allocation per array cost about 45 us each,
+// and one copy per table 50.)
+struct BaseLayout {
+    size_t rowptr, scale, blocks, wave, wmeta, grp, xchg, cnt, carry, tables, col, val, total;
+    BaseLayout(const pfr_csr* w, int64_t npad) {
+        const int64_t P = merge_wanted(w) ? merge_groups_bound(w) : 0, Q = P * pfr::kMergeWaves, M = w->M;
+        size_t at = 0;
+        auto take = [&](int64_t bytes) {
+            const size_t r = at;
+            at = (at + (size_t)bytes + 255) / 256 * 256;
+            return r;
+        };
+        rowptr = take(4 * (M + 1));
+        scale = take(w->vdt == PFR_I8 ? 4 * M : 0);
+        blocks = take(4 * (M + 1));
+        wave = take(P ? 8 * (Q + 1) : 0);
+        wmeta = take(16 * Q);
+        grp = take(16 * P);
+        xchg = take(8 * P);
+        cnt = take(4 * P);
+        carry = take(8 * P);
+        tables = at;
+        col = take(w->K > 65536 ? 4 * w->nnz : 2 * npad);
+        val = take((w->vdt == PFR_I8 ? 1 : 4) * npad);
+        total = at;
+    }
+};
+
+// Allocates the base arrays and sets their pointers (all but the merge-path
+// ones, which set_tables sets).
+void alloc_base(pfr_csr* w, const BaseLayout& L) {
+    PFR_HIP(hipMalloc(&w->base, L.total > 0 ? L.total : 256));
+    w->dev_bytes += (int64_t)L.total;
+    char* b = static_cast<char*>(w->base);
+    w->rowptr = reinterpret_cast<int32_t*>(b + L.rowptr);
+    if (w->vdt == PFR_I8) w->row_scale = reinterpret_cast<float*>(b + L.scale);
+    w->spmv_blocks = reinterpret_cast<int32_t*>(b + L.blocks);
+    if (w->K > 65536) w->col = reinterpret_cast<int32_t*>(b + L.col);
+    else w->col16 = reinterpret_cast<uint16_t*>(b + L.col);
+    w->val = b + L.val;
+}
+
+// Plans the row blocks and the merge-path partition and sends every table but
+// the row pointers; st holds at least L.tables bytes and is in use until the
+// stream has been synchronized.
+void set_tables(pfr_csr* w, const BaseLayout& L, const std::vector<int32_t>& rowptr, const float* row_scales,
+                Staging& st, hipStream_t s) {
+    char *h = st.p, *b = static_cast<char*>(w->base);
+    std::memset(h + L.scale, 0, L.tables - L.scale);
+    if (row_scales && w->M > 0) std::memcpy(h + L.scale, row_scales, 4 * (size_t)w->M);
+    const std::vector<int32_t> blocks = spmv_blocks(rowptr, w->M);  // at most M + 1
+    w->n_spmv_blocks = (int64_t)blocks.size() - 1;
+    std::memcpy(h + L.blocks, blocks.data(), 4 * blocks.size());
+    if (merge_wanted(w)) {
+        const MergePlan p = plan_merge(w, rowptr.data());
+        std::memcpy(h + L.wave, p.wave.data(), sizeof(int2) * p.wave.size());
+        std::memcpy(h + L.wmeta, p.wmeta.data(), sizeof(int4) * p.wmeta.size());
+        std::memcpy(h + L.grp, p.grp.data(), sizeof(int4) * p.grp.size());
+        w->mp_wave = reinterpret_cast<int2*>(b + L.wave);
+        w->mp_wmeta = reinterpret_cast<int4*>(b + L.wmeta);
+        w->mp_grp = reinterpret_cast<int4*>(b + L.grp);
+        w->mp_xchg = reinterpret_cast<unsigned long long*>(b + L.xchg);
+        w->mp_cnt = reinterpret_cast<uint32_t*>(b + L.cnt);
+        w->mp_carry = reinterpret_cast<float*>(b + L.carry);
+        w->mp_groups = (int32_t)p.P;
+    }
+    PFR_HIP(hipMemcpyAsync(b + L.scale, h + L.scale, L.tables - L.scale, hipMemcpyHostToDevice, s));
 }
 
 // ---- Build from a dense device weight ----------------------------------------
@@ -682,24 +830,36 @@ __device__ __forceinline__ void count_chunks(int32_t* s, uint64_t m, int64_t kw,
 // |v| > thr (the test of to_sparse, sparse_tensor.cpp:578; NaN fails it),
 // then its counts per sliced-ELL chunk (nchs of width kc) and per balanced
 // chunk (nchb of width kcw): cnt[r * (1 + nchs + nchb) + ...].
-__global__ __launch_bounds__(256) void k_dense_count(const float* __restrict__ D, int64_t K, float thr, int kc,
-                                                     int nchs, int kcw, int nchb, int32_t* __restrict__ cnt) {
+// mask, where given, multiplies D (apply_mask, sparse_tensor.cpp:616-631).
+template <bool MASK>
+__global__ __launch_bounds__(256) void k_dense_count(const float* __restrict__ D, const float* __restrict__ mask,
+                                                     int64_t K, float thr, int kc, int nchs, int kcw, int nchb,
+                                                     int32_t* __restrict__ cnt) {
     extern __shared__ int32_t sc[];  // [1 + nchs + nchb]
     const int n = 1 + nchs + nchb;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     for (int i = tid; i < n; i += 256) sc[i] = 0;
     __syncthreads();
     const float* row = D + (int64_t)blockIdx.x * K;
+    const float* mrow = MASK ? mask + (int64_t)blockIdx.x * K : nullptr;
     int tot = 0;
-    for (int64_t k0 = 0; k0 < K; k0 += 256) {
-        const int64_t k = k0 + tid;
-        const bool f = k < K && fabsf(row[k]) > thr;
-        const uint64_t m = __ballot(f);
-        if (lane == 0 && m) {
-            const int64_t kw = k0 + 64 * wave;
-            tot += (int)__popcll(m);
-            if (nchs) count_chunks(sc + 1, m, kw, kc);
-            if (nchb) count_chunks(sc + 1 + nchs, m, kw, kcw);
+    for (int64_t k0 = 0; k0 < K; k0 += 1024) {  // four loads ahead (clamped)
+        float v[4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            const int64_t k = min(k0 + 256 * u + tid, K - 1);
+            v[u] = row[k];
+            if constexpr (MASK) v[u] = v[u] * mrow[k];
+        }
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            const int64_t kw = k0 + 256 * u + 64 * wave;
+            const uint64_t m = __ballot(kw + lane < K && fabsf(v[u]) > thr);
+            if (lane == 0 && m) {
+                tot += (int)__popcll(m);
+                if (nchs) count_chunks(sc + 1, m, kw, kc);
+                if (nchb) count_chunks(sc + 1 + nchs, m, kw, kcw);
+            }
         }
     }
     if (lane == 0 && tot) atomicAdd(&sc[0], tot);
@@ -709,34 +869,56 @@ __global__ __launch_bounds__(256) void k_dense_count(const float* __restrict__ D
 
 // One workgroup per row of D: the kept entries in ascending column order at
 // rowptr[r] onward (the order to_sparse emits), as float values and the
-// columns as int32 (col) or uint16 (col16), whichever is given.
-__global__ __launch_bounds__(256) void k_dense_compact(const float* __restrict__ D, int64_t K, float thr,
-                                                       const int32_t* __restrict__ rowptr, int32_t* __restrict__ col,
+// columns as int32 (col) or uint16 (col16), whichever is given; mask as in
+// k_dense_count.  Row 0's workgroup also writes the padding after the nnz
+// entries (npad - nnz < 8 of them: value 0, column K).
+template <bool MASK>
+__global__ __launch_bounds__(256) void k_dense_compact(const float* __restrict__ D, const float* __restrict__ mask,
+                                                       int64_t K, float thr, const int32_t* __restrict__ rowptr,
+                                                       int64_t nnz, int64_t npad, int32_t* __restrict__ col,
                                                        uint16_t* __restrict__ col16, float* __restrict__ val) {
-    __shared__ int wsum[4];
+    __shared__ int wsum[16];  // [piece u of 256 columns][wave]
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const float* row = D + (int64_t)blockIdx.x * K;
+    const float* mrow = MASK ? mask + (int64_t)blockIdx.x * K : nullptr;
     int base = rowptr[blockIdx.x];
-    for (int64_t k0 = 0; k0 < K; k0 += 256) {
-        const int64_t k = k0 + tid;
-        const float v = k < K ? row[k] : 0.0f;
-        const bool f = k < K && fabsf(v) > thr;
-        const uint64_t m = __ballot(f);
-        if (lane == 0) wsum[wave] = (int)__popcll(m);
-        __syncthreads();
-        int off = base, total = 0;
+    if (blockIdx.x == 0 && nnz + tid < npad) {
+        val[nnz + tid] = 0.0f;
+        if (col16) col16[nnz + tid] = (uint16_t)(K < 65535 ? K : 65535);
+    }
+    for (int64_t k0 = 0; k0 < K; k0 += 1024) {
+        float v[4];
+        uint64_t m[4];
 #pragma unroll
-        for (int w = 0; w < 4; ++w) {
-            off += w < wave ? wsum[w] : 0;
-            total += wsum[w];
+        for (int u = 0; u < 4; ++u) {
+            const int64_t k = min(k0 + 256 * u + tid, K - 1);
+            v[u] = row[k];
+            if constexpr (MASK) v[u] = v[u] * mrow[k];
         }
-        if (f) {
-            const int j = off + (int)__popcll(m & ((uint64_t(1) << lane) - 1));
-            val[j] = v;
-            if (col) col[j] = (int32_t)k;
-            if (col16) col16[j] = (uint16_t)k;
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            m[u] = __ballot(k0 + 256 * u + tid < K && fabsf(v[u]) > thr);
+            if (lane == 0) wsum[4 * u + wave] = (int)__popcll(m[u]);
         }
-        base += total;
+        __syncthreads();
+        int off = base;
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            int at = off;
+#pragma unroll
+            for (int w = 0; w < 4; ++w) {
+                at += w < wave ? wsum[4 * u + w] : 0;
+                off += wsum[4 * u + w];
+            }
+            if (m[u] >> lane & 1) {
+                const int j = at + (int)__popcll(m[u] & ((uint64_t(1) << lane) - 1));
+                const int64_t k = k0 + 256 * u + tid;
+                val[j] = v[u];
+                if (col) col[j] = (int32_t)k;
+                if (col16) col16[j] = (uint16_t)k;
+            }
+        }
+        base = off;
         __syncthreads();
     }
 }
@@ -766,7 +948,7 @@ template <class CI, class V>
 __global__ __launch_bounds__(256) void k_sell_fill(int64_t npos, const int32_t* __restrict__ perm,
                                                    const int32_t* __restrict__ rowptr, const CI* __restrict__ col,
                                                    const V* __restrict__ val, const float* __restrict__ rs,
-                                                   const int64_t* __restrict__ off, int nch, int kc,
+                                                   const int32_t* __restrict__ soff, int nch, int kc,
                                                    int4* __restrict__ blk) {
     const int64_t i = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
     if (i >= npos) return;
@@ -779,7 +961,7 @@ __global__ __launch_bounds__(256) void k_sell_fill(int64_t npos, const int32_t* 
     for (int32_t j = b + lane; j < e; j += 64) {
         const int32_t k = (int32_t)col[j], c = k / kc;
         const int32_t step = j - first_at_least(col, b, j, c * kc);
-        int32_t* q = reinterpret_cast<int32_t*>(blk + off[sl * nch + c] + (step / 8) * 64 + 4 * r + (step % 8) / 2) +
+        int32_t* q = reinterpret_cast<int32_t*>(blk + soff[sl * (nch + 1) + c] + (step / 8) * 64 + 4 * r + (step % 8) / 2) +
                      (step % 2) * 2;
         q[0] = (k - c * kc) * 64;
         q[1] = __float_as_int(sizeof(V) == 1 ? (float)val[j] * scale : (float)val[j]);
@@ -1100,12 +1282,23 @@ __global__ __launch_bounds__(256) void k_pattern(int64_t M, const int32_t* __res
 
 // ---- Copies built on first use ----------------------------------------------
 
-// Each row's chunk index (column / width) does not decrease along it, which
-// the chunked copies' fills rely on (always true for ascending columns).
-bool chunks_ascend(const std::vector<int32_t>& rowptr, const std::vector<int32_t>& col, int64_t M, int64_t width) {
-    for (int64_t r = 0; r < M; ++r)
-        for (int32_t j = rowptr[(size_t)r] + 1; j < rowptr[(size_t)r + 1]; ++j)
-            if (col[(size_t)j] / width < col[(size_t)j - 1] / width) return false;
+// Counts each row's nonzeros per chunk of `width` columns (cnt[r * nch + c]).
+// False (cnt then unspecified) unless each row's chunk index does not decrease
+// along it, which the chunked copies' fills rely on (always true for ascending
+// columns).
+bool count_row_chunks(const std::vector<int32_t>& rowptr, const std::vector<int32_t>& col, int64_t M, int64_t width,
+                      int64_t nch, std::vector<int32_t>* cnt) {
+    cnt->assign((size_t)(M * nch), 0);
+    for (int64_t r = 0; r < M; ++r) {
+        int32_t* c = cnt->data() + r * nch;
+        int64_t lo = 0;  // first column of chunk c
+        for (int32_t j = rowptr[(size_t)r]; j < rowptr[(size_t)r + 1]; ++j) {
+            const int64_t k = col[(size_t)j];
+            if (k < lo) return false;
+            while (k >= lo + width) lo += width, ++c;
+            ++*c;
+        }
+    }
     return true;
 }
 
@@ -1138,18 +1331,17 @@ template <class CI, class V>
 void fill_sell(pfr_csr* w, const CI* col, hipStream_t s) {
     SellPlan p;
     if (!plan_sell(w->M, w->K, w->h_sell_cnt, &p)) return;
+    Staging st(w->ctx, sell_table_bytes(p));
     w->sell_blk = walloc<int4>(w, p.len + pfr::kSellTail);
     const int32_t pad = (int32_t)(p.kc * 64);
     fill_dev(w->sell_blk, p.len + pfr::kSellTail, make_int4(pad, 0, pad, 0), s);
-    if (w->sell_perm == nullptr) set_sell(w, p, s);  // else the fast copy's build uploaded them
-    int64_t* off = dev_alloc_copy(p.off.data(), (int64_t)p.off.size(), s);
+    if (w->sell_perm == nullptr) set_sell(w, p, st, s);  // else the fast copy's build uploaded them
     const int64_t npos = p.nslab * pfr::kSellRows;  // perm's length
     hipLaunchKernelGGL((k_sell_fill<CI, V>), dim3(waves_grid(npos)), dim3(256), 0, s, npos, w->sell_perm, w->rowptr,
-                       col, static_cast<const V*>(w->val), w->row_scale, off, (int)p.nch, (int)p.kc, w->sell_blk);
-    const hipError_t e = hipGetLastError();
-    (void)hipStreamSynchronize(s);
-    (void)hipFree(off);
-    if (e != hipSuccess) throw pfr::Error(PFR_ERR_HIP, std::string("k_sell_fill: ") + hipGetErrorString(e));
+                       col, static_cast<const V*>(w->val), w->row_scale, w->sell_soff, (int)p.nch, (int)p.kc,
+                       w->sell_blk);
+    PFR_HIP(hipGetLastError());
+    PFR_HIP(hipStreamSynchronize(s));
 }
 
 // The fast mode's sliced-ELL copy: the same plan and tables (uploaded here
@@ -1161,7 +1353,8 @@ void fill_sell_fast(pfr_csr* w, const CI* col, hipStream_t s) {
     w->sell_blk_fast = walloc<int4>(w, p.len + pfr::kSellTail);
     const int32_t pad = (int32_t)(p.kc * 64);
     fill_dev(w->sell_blk_fast, p.len + pfr::kSellTail, make_int4(pad, 0, pad, 0), s);
-    if (w->sell_perm == nullptr) set_sell(w, p, s);
+    Staging st(w->ctx, sell_table_bytes(p));
+    if (w->sell_perm == nullptr) set_sell(w, p, st, s);
     const int64_t nthr = p.nslab * 4 * p.nch;
     hipLaunchKernelGGL(k_sell_fill_fast<CI>, dim3((unsigned)((nthr + 255) / 256)), dim3(256), 0, s, nthr,
                        (int)p.nch, (int)p.kc, w->sell_perm, w->rowptr, col, static_cast<const float*>(w->val),
@@ -1270,7 +1463,8 @@ void drop_copy(pfr_csr* w, uint32_t bit) {
     if (bit == pfr::kCopySell || bit == pfr::kCopySellFast) {
         free_null(bit == pfr::kCopySell ? w->sell_blk : w->sell_blk_fast);
         if (w->sell_blk == nullptr && w->sell_blk_fast == nullptr) {  // the tables serve neither copy now
-            free_null(w->sell_perm), free_null(w->sell_soff);
+            free_null(w->sell_perm);
+            w->sell_soff = nullptr;
             w->sell_nslab = w->sell_nch = w->sell_kc = 0;
             w->sell_len = 0;
         }
@@ -1294,6 +1488,9 @@ void drop_copy(pfr_csr* w, uint32_t bit) {
 pfr_csr* build(pfr_ctx* ctx, int64_t M, int64_t K, const std::vector<int32_t>& rowptr,
                const std::vector<int32_t>& col, const void* vals, pfr_dtype vdt,
                const float* row_scales) {
+    static const char zeros[32] = {};
+    std::vector<uint16_t> c16;
+    Staging st;  // both outlive the copies from them, a failed build's too
     auto* w = new pfr_csr();
     try {
         w->ctx = ctx;
@@ -1305,35 +1502,29 @@ pfr_csr* build(pfr_ctx* ctx, int64_t M, int64_t K, const std::vector<int32_t>& r
         for (int64_t r = 0; r < M; ++r) mx = std::max(mx, rowptr[r + 1] - rowptr[r]);
         w->max_row_nnz = mx;
         hipStream_t s = ctx->stream;
-        w->rowptr = walloc_copy(w, rowptr.data(), M + 1, s);
         // col16 and val hold whole records of four and one spare record;
         // padding entries are value 0 at column K (x's zero slot in the
         // merge-path kernels, which read whole records and point loads past
         // a share at the spare one)
         const int64_t npad = (w->nnz + 3) / 4 * 4 + 4;
+        const BaseLayout L(w, npad);
+        alloc_base(w, L);
+        st = Staging(ctx, L.tables);
+        std::memcpy(st.p + L.rowptr, rowptr.data(), 4 * (size_t)(M + 1));
+        PFR_HIP(hipMemcpyAsync(w->rowptr, st.p + L.rowptr, 4 * (size_t)(M + 1), hipMemcpyHostToDevice, s));
         if (K > 65536) {
-            w->col = walloc_copy(w, col.data(), w->nnz, s);
+            if (w->nnz > 0)
+                PFR_HIP(hipMemcpyAsync(w->col, col.data(), 4 * (size_t)w->nnz, hipMemcpyHostToDevice, s));
         } else {  // allocated (padding only) also without entries: kernels may load a row's first record
-            std::vector<uint16_t> c16(col.begin(), col.end());
+            c16.assign(col.begin(), col.end());
             c16.resize((size_t)npad, (uint16_t)std::min<int64_t>(K, 65535));
-            w->col16 = walloc_copy(w, c16.data(), npad, s);
-            PFR_HIP(hipStreamSynchronize(s));  // c16 goes out of scope
+            PFR_HIP(hipMemcpyAsync(w->col16, c16.data(), 2 * (size_t)npad, hipMemcpyHostToDevice, s));
         }
-        if (vdt == PFR_F32) {
-            std::vector<float> v(static_cast<const float*>(vals), static_cast<const float*>(vals) + w->nnz);
-            v.resize((size_t)npad, 0.0f);
-            w->val = walloc_copy(w, v.data(), npad, s);
-            PFR_HIP(hipStreamSynchronize(s));
-        } else {
-            std::vector<int8_t> v(static_cast<const int8_t*>(vals), static_cast<const int8_t*>(vals) + w->nnz);
-            v.resize((size_t)npad, 0);
-            w->val = walloc_copy(w, v.data(), npad, s);
-            PFR_HIP(hipStreamSynchronize(s));
-        }
-        if (row_scales) w->row_scale = walloc_copy(w, row_scales, M, s);
-        std::vector<int32_t> blocks = spmv_blocks(rowptr, M);
-        w->n_spmv_blocks = (int64_t)blocks.size() - 1;
-        w->spmv_blocks = walloc_copy(w, blocks.data(), (int64_t)blocks.size(), s);
+        const size_t vb = vdt == PFR_I8 ? 1 : 4;
+        if (w->nnz > 0) PFR_HIP(hipMemcpyAsync(w->val, vals, vb * (size_t)w->nnz, hipMemcpyHostToDevice, s));
+        PFR_HIP(hipMemcpyAsync(static_cast<char*>(w->val) + vb * (size_t)w->nnz, zeros, vb * (size_t)(npad - w->nnz),
+                               hipMemcpyHostToDevice, s));
+        set_tables(w, L, rowptr, row_scales, st, s);
         bool sorted = true;
         for (int64_t r = 0; r < M && sorted; ++r)
             for (int32_t j = rowptr[r] + 1; j < rowptr[r + 1]; ++j)
@@ -1343,19 +1534,10 @@ pfr_csr* build(pfr_ctx* ctx, int64_t M, int64_t K, const std::vector<int32_t>& r
         int64_t kc, nchs, nchb = 0, kcw = 1;
         sell_geom(K, &kc, &nchs);
         std::vector<int32_t> cs, cb;
-        if (sell_wanted(M, K, w->nnz) && chunks_ascend(rowptr, col, M, kc)) {
-            cs.assign((size_t)(M * nchs), 0);
-            for (int64_t r = 0; r < M; ++r)
-                for (int32_t j = rowptr[r]; j < rowptr[r + 1]; ++j) ++cs[(size_t)(r * nchs + col[j] / kc)];
-        }
-        if (w->nnz > 0 && bal_geom(K, &nchb, &kcw) && chunks_ascend(rowptr, col, M, kcw)) {
-            cb.assign((size_t)(M * nchb), 0);
-            for (int64_t r = 0; r < M; ++r)
-                for (int32_t j = rowptr[r]; j < rowptr[r + 1]; ++j) ++cb[(size_t)(r * nchb + col[j] / kcw)];
-        }
+        if (!sell_wanted(M, K, w->nnz) || !count_row_chunks(rowptr, col, M, kc, nchs, &cs)) cs.clear();
+        if (w->nnz == 0 || !bal_geom(K, &nchb, &kcw) || !count_row_chunks(rowptr, col, M, kcw, nchb, &cb)) cb.clear();
         set_lazy(w, rowptr, std::move(cs), std::move(cb));
-        set_merge(w, rowptr, s);
-        PFR_HIP(hipStreamSynchronize(s));
+        PFR_HIP(hipStreamSynchronize(s));  // the host buffers go out of scope
         return w;
     } catch (...) {
         (void)hipStreamSynchronize(ctx->stream);
@@ -1364,11 +1546,12 @@ pfr_csr* build(pfr_ctx* ctx, int64_t M, int64_t K, const std::vector<int32_t>& r
     }
 }
 
-// The handle of D (M x K, row-major, device), as build() makes it from the
-// same entries: counts on the device, copied back (M x a few integers) for
-// the row pointers and the copies' plans, then the entries compacted on the
-// device, so the nonzeros never leave the GPU.
-pfr_csr* build_dense_dev(pfr_ctx* ctx, const float* D, int64_t M, int64_t K, float thr) {
+// The handle of D * mask (M x K, row-major, device; mask may be null), as
+// build() makes it from the same entries: counts on the device, copied back (M
+// x a few integers) for the row pointers and the copies' plans, then the
+// entries compacted on the device while the host plans the tables, so the
+// nonzeros never leave the GPU.
+pfr_csr* build_dense_dev(pfr_ctx* ctx, const float* D, const float* mask, int64_t M, int64_t K, float thr) {
     hipStream_t s = ctx->stream;
     int64_t kc, nchs;
     sell_geom(K, &kc, &nchs);
@@ -1376,21 +1559,36 @@ pfr_csr* build_dense_dev(pfr_ctx* ctx, const float* D, int64_t M, int64_t K, flo
     int64_t nchb = 0, kcw = 1;
     if (!bal_geom(K, &nchb, &kcw)) nchb = 0, kcw = 1;
     const int64_t stride = 1 + nchs + nchb;
-    std::vector<int32_t> cnt((size_t)(M * stride));
+    std::vector<int32_t> rowptr((size_t)M + 1, 0), cs, cb;
+    int32_t mx = 0;
     {
-        DevTmp dcnt(sizeof(int32_t) * (size_t)(M * stride));
-        hipLaunchKernelGGL(k_dense_count, dim3((unsigned)M), dim3(256), (size_t)stride * 4, s, D, K, thr, (int)kc,
-                           (int)nchs, (int)kcw, (int)nchb, dcnt.as<int32_t>());
+        const size_t bytes = sizeof(int32_t) * (size_t)(M * stride);
+        Staging st(ctx, bytes);
+        std::unique_ptr<DevTmp> tmp;
+        if (!st.lock.owns_lock()) tmp.reset(new DevTmp(bytes));  // another thread's build has the context's buffer
+        int32_t* dcnt = tmp ? tmp->as<int32_t>() : static_cast<int32_t*>(ctx->scratch[6].ensure(bytes));
+        if (mask)
+            hipLaunchKernelGGL(k_dense_count<true>, dim3((unsigned)M), dim3(256), (size_t)stride * 4, s, D, mask, K, thr,
+                               (int)kc, (int)nchs, (int)kcw, (int)nchb, dcnt);
+        else
+            hipLaunchKernelGGL(k_dense_count<false>, dim3((unsigned)M), dim3(256), (size_t)stride * 4, s, D, mask, K,
+                               thr, (int)kc, (int)nchs, (int)kcw, (int)nchb, dcnt);
         PFR_HIP(hipGetLastError());
-        PFR_HIP(hipMemcpyAsync(cnt.data(), dcnt.p, cnt.size() * 4, hipMemcpyDeviceToHost, s));
+        PFR_HIP(hipMemcpyAsync(st.p, dcnt, bytes, hipMemcpyDeviceToHost, s));
         PFR_HIP(hipStreamSynchronize(s));
+        const auto* cnt = reinterpret_cast<const int32_t*>(st.p);
+        if (nchs > 0) cs.resize((size_t)(M * nchs));
+        if (nchb > 0) cb.resize((size_t)(M * nchb));
+        for (int64_t r = 0; r < M; ++r) {
+            const int32_t* c = cnt + r * stride;
+            pfr::require((int64_t)rowptr[(size_t)r] + c[0] < INT32_MAX, "nnz exceeds 32-bit indices");
+            rowptr[(size_t)r + 1] = rowptr[(size_t)r] + c[0];
+            mx = std::max(mx, c[0]);
+            std::copy(c + 1, c + 1 + nchs, cs.begin() + r * nchs);
+            std::copy(c + 1 + nchs, c + stride, cb.begin() + r * nchb);
+        }
     }
-    std::vector<int32_t> rowptr((size_t)M + 1, 0), len((size_t)M);
-    for (int64_t r = 0; r < M; ++r) {
-        len[(size_t)r] = cnt[(size_t)(r * stride)];
-        pfr::require((int64_t)rowptr[(size_t)r] + len[(size_t)r] < INT32_MAX, "nnz exceeds 32-bit indices");
-        rowptr[(size_t)r + 1] = rowptr[(size_t)r] + len[(size_t)r];
-    }
+    Staging st;  // outlives the copies from it, a failed build's too
     auto* w = new pfr_csr();
     try {
         w->ctx = ctx;
@@ -1398,40 +1596,26 @@ pfr_csr* build_dense_dev(pfr_ctx* ctx, const float* D, int64_t M, int64_t K, flo
         w->K = K;
         w->nnz = rowptr[(size_t)M];
         w->vdt = PFR_F32;
-        w->max_row_nnz = M ? *std::max_element(len.begin(), len.end()) : 0;
+        w->max_row_nnz = mx;
         w->cols_sorted = true;
-        w->rowptr = walloc_copy(w, rowptr.data(), M + 1, s);
         const int64_t npad = (w->nnz + 3) / 4 * 4 + 4;  // whole records and a spare one, as build() pads
-        float* val = walloc<float>(w, npad);
-        w->val = val;
-        fill_dev(val + w->nnz, npad - w->nnz, 0.0f, s);
-        if (K > 65536) {
-            w->col = walloc<int32_t>(w, w->nnz);
-        } else {
-            w->col16 = walloc<uint16_t>(w, npad);
-            fill_dev(w->col16 + w->nnz, npad - w->nnz, (uint16_t)std::min<int64_t>(K, 65535), s);
-        }
-        hipLaunchKernelGGL(k_dense_compact, dim3((unsigned)M), dim3(256), 0, s, D, K, thr, w->rowptr, w->col,
-                           w->col16, val);
+        const BaseLayout L(w, npad);
+        alloc_base(w, L);
+        st = Staging(ctx, L.tables);
+        std::memcpy(st.p + L.rowptr, rowptr.data(), 4 * (size_t)(M + 1));
+        PFR_HIP(hipMemcpyAsync(w->rowptr, st.p + L.rowptr, 4 * (size_t)(M + 1), hipMemcpyHostToDevice, s));
+        if (mask)
+            hipLaunchKernelGGL(k_dense_compact<true>, dim3((unsigned)M), dim3(256), 0, s, D, mask, K, thr, w->rowptr,
+                               w->nnz, npad, w->col, w->col16, static_cast<float*>(w->val));
+        else
+            hipLaunchKernelGGL(k_dense_compact<false>, dim3((unsigned)M), dim3(256), 0, s, D, mask, K, thr, w->rowptr,
+                               w->nnz, npad, w->col, w->col16, static_cast<float*>(w->val));
         PFR_HIP(hipGetLastError());
-        std::vector<int32_t> blocks = spmv_blocks(rowptr, M);
-        w->n_spmv_blocks = (int64_t)blocks.size() - 1;
-        w->spmv_blocks = walloc_copy(w, blocks.data(), (int64_t)blocks.size(), s);
-        PFR_HIP(hipStreamSynchronize(s));  // blocks goes out of scope
-        if (w->nnz == 0) return w;
-        std::vector<int32_t> cs, cb;
-        if (nchs > 0 && sell_wanted(M, K, w->nnz)) {
-            cs.resize((size_t)(M * nchs));
-            for (int64_t r = 0; r < M; ++r)
-                std::copy(cnt.begin() + r * stride + 1, cnt.begin() + r * stride + 1 + nchs, cs.begin() + r * nchs);
+        set_tables(w, L, rowptr, nullptr, st, s);
+        if (w->nnz > 0) {
+            if (!sell_wanted(M, K, w->nnz)) cs.clear();
+            set_lazy(w, rowptr, std::move(cs), std::move(cb));
         }
-        if (nchb > 0) {
-            cb.resize((size_t)(M * nchb));
-            for (int64_t r = 0; r < M; ++r)
-                std::copy(cnt.begin() + r * stride + 1 + nchs, cnt.begin() + (r + 1) * stride, cb.begin() + r * nchb);
-        }
-        set_lazy(w, rowptr, std::move(cs), std::move(cb));
-        set_merge(w, rowptr, s);
         PFR_HIP(hipStreamSynchronize(s));
         return w;
     } catch (...) {
@@ -1594,23 +1778,19 @@ int pfr_csr_from_dense_dev(pfr_ctx* ctx, const float* dense, int64_t rows, int64
         hipStream_t s = ctx->stream;
         const float* D = dense;
         std::unique_ptr<DevTmp> tmp;
-        if (transpose || mask) {  // op(dense * mask), row-major
+        if (transpose) {  // op(dense * mask), row-major; else the mask is applied as the entries are read
             tmp.reset(new DevTmp(sizeof(float) * (size_t)(M * K)));
-            if (transpose) {
-                const unsigned tiles = (unsigned)((rows + 31) / 32 * ((cols + 31) / 32));
-                if (mask)
-                    hipLaunchKernelGGL(k_transpose_mask<true>, dim3(tiles), dim3(256), 0, s, dense, mask, rows, cols,
-                                       tmp->as<float>());
-                else
-                    hipLaunchKernelGGL(k_transpose_mask<false>, dim3(tiles), dim3(256), 0, s, dense, mask, rows,
-                                       cols, tmp->as<float>());
-                PFR_HIP(hipGetLastError());
-            } else {
-                pfr::apply_mask_dev(s, dense, mask, M * K, tmp->as<float>());
-            }
+            const unsigned tiles = (unsigned)((rows + 31) / 32 * ((cols + 31) / 32));
+            if (mask)
+                hipLaunchKernelGGL(k_transpose_mask<true>, dim3(tiles), dim3(256), 0, s, dense, mask, rows, cols,
+                                   tmp->as<float>());
+            else
+                hipLaunchKernelGGL(k_transpose_mask<false>, dim3(tiles), dim3(256), 0, s, dense, mask, rows, cols,
+                                   tmp->as<float>());
+            PFR_HIP(hipGetLastError());
             D = tmp->as<float>();
         }
-        *out = build_dense_dev(ctx, D, M, K, threshold);
+        *out = build_dense_dev(ctx, D, transpose ? nullptr : mask, M, K, threshold);
         PFR_HIP(hipStreamSynchronize(s));  // tmp is freed on return
     });
 }
