@@ -1932,7 +1932,8 @@ __global__ __launch_bounds__((sell_threads<XVEC, W, XT>())) void k_spmm_sell(
     const int slab = __builtin_amdgcn_readfirstlane((int)blockIdx.x * W + wave);
     const int n0 = (int)blockIdx.y * pfr::kSellCols;
     const int bufq = (kc + 1) * 4;  // float4 per buffer
-    if (tid < 8) xs[(tid >> 2) * bufq + kc * 4 + (tid & 3)] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+    // (a single chunk has one buffer)
+    if (tid < (nch > 1 ? 8 : 4)) xs[(tid >> 2) * bufq + kc * 4 + (tid & 3)] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
     float a0 = 0.0f, a1 = 0.0f, a2 = 0.0f, a3 = 0.0f;
 
     // Load i of this wave for chunk c: rows 16j .. 16j+15 of the chunk, lane
@@ -2137,7 +2138,7 @@ void launch_sell_w(pfr_ctx* ctx, const pfr_csr* Wt, const float* X, int N, int64
                    int64_t ldy_r, int64_t ldy_c, int yvec, const float* bias, int64_t c_size, float beta, int act,
                    float alpha) {
     auto kern = k_spmm_sell<FAST, XVEC, W, XT>;
-    const size_t lds = (size_t)(Wt->sell_kc + 1) * 64 * 2;
+    const size_t lds = (size_t)(Wt->sell_kc + 1) * 64 * (Wt->sell_nch > 1 ? 2 : 1);
     // more than 64 KiB of dynamic LDS has to be allowed per kernel and device
     static uint64_t allowed = 0;  // bit d: done on device d (< 64)
     const uint64_t bit = ctx->device < 64 ? (uint64_t(1) << ctx->device) : 0;
