@@ -105,10 +105,14 @@ __global__ __launch_bounds__(256) void k_add(const float* __restrict__ a, const 
 }
 
 // LayerNormalization with the rows staged in LDS: the block loads `rows`
-// rows coalesced, one lane per row then runs the reference's sequential
-// mean and variance over its LDS row (same operations in the same order as
-// nn.cpp:457-470), and the whole block writes the normalised rows.  LDS:
-// rows * stride floats (stride a multiple of 4, padded by 4 so the lanes'
+// rows coalesced, one lane per row runs the reference's sequential mean, the
+// whole block turns its elements into differences from it, one lane per row
+// adds their squares in order (same operations in the same order as
+// nn.cpp:457-470), and the whole block writes the normalised rows from the
+// differences.  The two chains of `norm` dependent adds bound it:
+// 1024 x 768 takes 15.2 us (20.3 with the subtractions in the second chain's
+// lane).
+// LDS: rows * stride floats (stride a multiple of 4, padded by 4 so the lanes'
 // 16-byte reads fall in different banks), then the rows' means and inverse
 // standard deviations.
 constexpr int kLnThreads = 256;
@@ -126,70 +130,55 @@ __global__ __launch_bounds__(kLnThreads) void k_layernorm_lds(const float* __res
         for (int i = threadIdx.x; i < norm; i += kLnThreads) lds[j * stride + i] = xr[i];
     }
     __syncthreads();
-    if ((int)threadIdx.x < rows) {
-        const float* row = lds + threadIdx.x * stride;
-        // in element order, 32 at a time: the next 32 are read from LDS into
-        // the other register set while the current 32 are added, so the
-        // dependent adds do not wait on each read
+    // term(v) summed over an LDS row in element order, 32 at a time: the next
+    // 32 are read into the other register set while the current 32 are
+    // added, so the dependent adds do not wait on each read
+    auto sum = [&](const float* row, auto term) {
         const int n32 = norm & ~31;
+        float s = 0.0f;
+        float4 va[8], vb[8];
         auto rd = [&](int i, float4* v) {
 #pragma unroll
             for (int k = 0; k < 8; ++k) v[k] = *reinterpret_cast<const float4*>(row + i + 4 * k);
         };
-        float4 va[8], vb[8];
-        float mean = 0.0f;
-        auto add_sum = [&](const float4* v) {
+        auto add = [&](const float4* v) {
 #pragma unroll
             for (int k = 0; k < 8; ++k) {
-                mean = mean + v[k].x;
-                mean = mean + v[k].y;
-                mean = mean + v[k].z;
-                mean = mean + v[k].w;
+                s = s + term(v[k].x);
+                s = s + term(v[k].y);
+                s = s + term(v[k].z);
+                s = s + term(v[k].w);
             }
         };
         if (n32) rd(0, va);
         for (int i = 0; i < n32; i += 64) {
             if (i + 32 < n32) rd(i + 32, vb);
-            add_sum(va);
+            add(va);
             if (i + 32 >= n32) break;
             if (i + 64 < n32) rd(i + 64, va);
-            add_sum(vb);
+            add(vb);
         }
-        for (int i = n32; i < norm; ++i) mean = mean + row[i];
-        mean = mean / (float)norm;
-        float var = 0.0f;
-        auto add_var = [&](const float4* v) {
-#pragma unroll
-            for (int k = 0; k < 8; ++k) {
-                const float d0 = v[k].x - mean, d1 = v[k].y - mean, d2 = v[k].z - mean, d3 = v[k].w - mean;
-                var = var + d0 * d0;
-                var = var + d1 * d1;
-                var = var + d2 * d2;
-                var = var + d3 * d3;
-            }
-        };
-        if (n32) rd(0, va);
-        for (int i = 0; i < n32; i += 64) {
-            if (i + 32 < n32) rd(i + 32, vb);
-            add_var(va);
-            if (i + 32 >= n32) break;
-            if (i + 64 < n32) rd(i + 64, va);
-            add_var(vb);
-        }
-        for (int i = n32; i < norm; ++i) {
-            const float d = row[i] - mean;
-            var = var + d * d;
-        }
-        var = var / (float)norm;
-        stat[threadIdx.x] = mean;
+        for (int i = n32; i < norm; ++i) s = s + term(row[i]);
+        return s;
+    };
+    if ((int)threadIdx.x < rows)
+        stat[threadIdx.x] = sum(lds + threadIdx.x * stride, [](float v) { return v; }) / (float)norm;
+    __syncthreads();
+    for (int j = 0; j < rows; ++j) {
+        const float mean = stat[j];
+        for (int i = threadIdx.x; i < norm; i += kLnThreads) lds[j * stride + i] = lds[j * stride + i] - mean;
+    }
+    __syncthreads();
+    if ((int)threadIdx.x < rows) {
+        const float var = sum(lds + threadIdx.x * stride, [](float d) { return d * d; }) / (float)norm;
         stat[rpb + threadIdx.x] = 1.0f / sqrtf(var + eps);
     }
     __syncthreads();
     for (int j = 0; j < rows; ++j) {
-        const float mean = stat[j], inv_std = stat[rpb + j];
+        const float inv_std = stat[rpb + j];
         float* yr = y + (r0 + j) * norm;
         for (int i = threadIdx.x; i < norm; i += kLnThreads)
-            yr[i] = scale[i] * (lds[j * stride + i] - mean) * inv_std + bias[i];
+            yr[i] = scale[i] * lds[j * stride + i] * inv_std + bias[i];
     }
 }
 

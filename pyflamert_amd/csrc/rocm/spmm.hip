@@ -2108,11 +2108,16 @@ __global__ __launch_bounds__((sell_threads<XVEC, W, XT>())) void k_spmm_sell(
                 *reinterpret_cast<float4*>(yr + cn) = make_float4(a0, a1, a2, a3);
             } else {
                 const float a[4] = {a0, a1, a2, a3};
+                // a bias of one element per feature (the usual Gemm's) is the
+                // row's, without a division per output
+                const bool brow = bias != nullptr && ldy_r == 1 && c_size == ldy_c;
+                const float* const brp = brow ? bias + row : nullptr;
 #pragma unroll
                 for (int i = 0; i < 4; ++i)
                     if (cn + i < N) {
                         const int64_t f = (int64_t)row * ldy_r + (int64_t)(cn + i) * ldy_c;
-                        Y[f] = bias_add(a[i], f, bias, c_size, beta, act);
+                        Y[f] = brow ? pfr::bias_add_at(a[i], brp, beta, act)
+                                    : bias_add(a[i], f, bias, c_size, beta, act);
                     }
             }
         }
@@ -2177,7 +2182,9 @@ void launch_sell_x(pfr_ctx* ctx, const pfr_csr* Wt, const float* X, int N, int64
     launch_sell_w<FAST, XVEC, WV, XT>(ctx, Wt, X, N, ldx, nx, Y, ldy_r, ldy_c, yvec, bias, c_size, beta, act, alpha)
     const int w = sell_waves(ctx, Wt, N);
     if (w == 16) PFR_SELLW(16);
+    else if (w == 12) PFR_SELLW(12);
     else if (w == 8) PFR_SELLW(8);
+    else if (w == 6) PFR_SELLW(6);
     else PFR_SELLW(4);
 #undef PFR_SELLW
 }
