@@ -66,8 +66,9 @@ __device__ __forceinline__ int32_t f2i_trunc_x86(float r) {
 // logistic function of 2 u.  It has no cancellation at u << 0 (where the
 // reference's 1 + tanhf(u) keeps an ulp of 1), the same limits (-0 for large
 // negative v, NaN for -inf and NaN), and costs about half of the device's
-// tanhf, which took a fifth of the 3072 x 768 product's launch in its epilogue
-// (1024 tokens, 57 -> 50 us with the row bias of k_spmm_sell).
+// tanhf, which with a division per bias index took a quarter of the 3072 x 768
+// product's launch on 1024 tokens (57 -> 44 us with the other epilogue change and
+// one LDS buffer, see k_spmm_sell).
 __device__ __forceinline__ float gelu(float v) {
     const float inner = 0.7978845608028654f * (v + 0.044715f * v * v * v);
     return v * __builtin_amdgcn_rcpf(1.0f + expf(-2.0f * inner));

@@ -1913,8 +1913,8 @@ constexpr int sell_threads() { return 64 * (W + (sell_stager<XVEC, W, XT>() ? 1 
 // row-major, rows ldx floats apart, 16-byte aligned, K % 4 == 0): each
 // chunk is staged from A's rows through registers into the same LDS layout,
 // scaled by alpha when `scale` (RN(alpha * a), the operand the reference's
-// Gemm multiplies), so no transposed copy is written first.  The 16-wave
-// launch stages every chunk with all its waves; the 4- and 8-wave launches
+// Gemm multiplies), so no transposed copy is written first.  The 12- and
+// 16-wave launches stage every chunk with all their waves; the 4- and 8-wave launches
 // take it only for one chunk, staged by all their waves.
 template <bool FAST, bool XVEC, int W, bool XT>
 __global__ __launch_bounds__((sell_threads<XVEC, W, XT>())) void k_spmm_sell(
@@ -2160,16 +2160,21 @@ void launch_sell_w(pfr_ctx* ctx, const pfr_csr* Wt, const float* X, int N, int64
 
 // Waves per workgroup of the column-slice launch for N columns, and its
 // rounds.  One workgroup runs per CU (its LDS takes most of the CU), so the
-// launch takes ceil(workgroups / CUs) rounds.  A round of 4-, 8- and 16-wave
-// workgroups takes about 1 : 1.30 : 2.14 (measured on the 4096 x 4096, 10 %
-// weight at N = 64, 128 and 256, one round each); the wave count with the
-// fewest estimated clocks runs, the larger on a tie.  Fewer than four waves
-// lose: each wave then stages more of X than it walks.
+// launch takes ceil(workgroups / CUs) rounds.  A round of 4-, 8-, 12- and
+// 16-wave workgroups takes about 1 : 1.30 : 1.74 : 2.14 (measured on the 4096 x
+// 4096, 10 % weight at N = 64, 128, 128 and 256, one round each); the wave
+// count with the fewest estimated clocks runs, the larger on a tie.  (12 waves
+// fill the chip where 16 leave a quarter of it idle, 8 need a second round:
+// 3001 x 5003 on 256 columns 48.0 -> 41.5 us, 768 x 3072 on 1024 53.0 -> 48.2,
+// 768 x 768 on 1024 15.4 -> 13.5.)  The same rule holds for a weight of one
+// chunk, several of whose workgroups share a CU.  Fewer than four waves lose:
+// each wave then stages more of X than it walks.
 int sell_waves(const pfr_ctx* ctx, const pfr_csr* Wt, int64_t N, int64_t* rounds_out = nullptr) {
     const int64_t slices = (N + pfr::kSellCols - 1) / pfr::kSellCols;
     auto rounds = [&](int64_t w) { return ((Wt->sell_nslab + w - 1) / w * slices + ctx->num_cu - 1) / ctx->num_cu; };
-    const int64_t c16 = rounds(16) * 214, c8 = rounds(8) * 130, c4 = rounds(4) * 100;
-    const int w = (c16 <= c8 && c16 <= c4) ? 16 : (c8 <= c4 ? 8 : 4);
+    const int64_t c16 = rounds(16) * 214, c12 = rounds(12) * 174, c8 = rounds(8) * 130, c4 = rounds(4) * 100;
+    const int64_t best = std::min(std::min(c16, c12), std::min(c8, c4));
+    const int w = best == c16 ? 16 : (best == c12 ? 12 : (best == c8 ? 8 : 4));
     if (rounds_out) *rounds_out = rounds(w);
     return w;
 }
@@ -2184,7 +2189,6 @@ void launch_sell_x(pfr_ctx* ctx, const pfr_csr* Wt, const float* X, int N, int64
     if (w == 16) PFR_SELLW(16);
     else if (w == 12) PFR_SELLW(12);
     else if (w == 8) PFR_SELLW(8);
-    else if (w == 6) PFR_SELLW(6);
     else PFR_SELLW(4);
 #undef PFR_SELLW
 }
@@ -2381,13 +2385,13 @@ bool sell_serves(const pfr_csr* W, int64_t N, bool fast) {
            N < (int64_t)pfr::kSellCols * 65535;
 }
 
-// Its launch for N columns runs in one round, with 16-wave workgroups or,
-// for a single chunk, 4 or 8 (their chunk 0 is staged by every wave; later
+// Its launch for N columns runs in one round, with 12- or 16-wave workgroups
+// or, for a single chunk, 4 or 8 (their chunk 0 is staged by every wave; later
 // chunks would fall to the staging wave alone).
 bool sell_one_round(const pfr_ctx* ctx, const pfr_csr* W, int64_t N) {
     int64_t rounds = 0;
     const int w = sell_waves(ctx, W, N, &rounds);
-    return rounds == 1 && (w == 16 || W->sell_nch == 1);
+    return rounds == 1 && (w >= 12 || W->sell_nch == 1);
 }
 
 // Launch the kernel that fits N.  Output (row, c) -> Y[row*ldy_r + c*ldy_c].
