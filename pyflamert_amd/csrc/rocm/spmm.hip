@@ -2438,8 +2438,7 @@ void check_act(int act) {
 // when the handle still has it pending (its first such product).
 void ensure_copies(const pfr_ctx* ctx, const pfr_csr* W, int64_t N, bool fast) {
     uint32_t need = 0;
-    // (an int8 weight has the storage-order copy only, for both modes)
-    if (N >= kSellMinN) need |= fast && W->vdt != PFR_I8 ? pfr::kCopySellFast : pfr::kCopySell;
+    if (N >= kSellMinN) need |= fast ? pfr::kCopySellFast : pfr::kCopySell;
     if (fast && ((N >= 2 && N <= 8) || (N == 1 && !(ctx->merge && W->mp_wave != nullptr)))) need |= pfr::kCopyBal;
     if (!fast && N <= 8) need |= pfr::kCopyChain;
     if ((W->pending.load(std::memory_order_acquire) & need) != 0) pfr::csr_build_copies(const_cast<pfr_csr*>(W), need);
