@@ -1687,11 +1687,25 @@ __device__ __forceinline__ void static_for(F&& f) {
     }
 }
 
-template <int W>
-constexpr int sell_loads_per_iter() {
-    // a chunk's 16-row loads per wave, spread over about three iterations of
-    // the walk (four groups each); the rest are issued after the walk
-    return (pfr::kSellMaxKC / 16 / W + 2) / 3;
+// Where the non-finite rule (k_nonfinite_fix) makes outputs NaN in one slab and
+// 16-column slice: bit i for column n0 + 4 q + i of the lane's row.  X is the
+// transposed activation; the wave reads 64 consecutive k of a column at once.
+__device__ __forceinline__ int sell_nonfinite(const float* X, int64_t ldx, int n0, int N, int K,
+                                                        float alpha, int scale, const uint64_t* bm, int64_t nw,
+                                                        int row, int q) {
+    const int lane = (int)threadIdx.x & 63, nc = min(pfr::kSellCols, N - n0);
+    int hit = 0;
+    for (int k0 = 0; k0 < K; k0 += 64)
+#pragma unroll 1
+        for (int c = 0; c < nc; ++c) {
+            float v = k0 + lane < K ? X[(int64_t)(n0 + c) * ldx + k0 + lane] : 0.0f;
+            if (scale && k0 + lane < K) v = alpha * v;
+            const bool nan = __ballot(v != v) != 0;
+            const uint64_t inf = __ballot(__builtin_isinf(v));
+            if (!nan && inf == 0) continue;
+            if (c >> 2 == q && row >= 0 && (nan || (inf & ~bm[row * nw + (k0 >> 6)]) != 0)) hit |= 1 << (c & 3);
+        }
+    return hit;
 }
 
 using lds_char = __attribute__((address_space(3))) char;
@@ -1701,19 +1715,10 @@ using lds_char = __attribute__((address_space(3))) char;
 // iteration, each reloaded with the group four ahead as soon as it is used
 // (so loads run three groups ahead), past the run's end into the next run or
 // the tail, and never used there; a last partial iteration uses what is
-// already loaded.  xb is the lane's view of the chunk's X rows.  With MORE,
-// the walk also copies DPI 16-row blocks of the next chunk per iteration
-// into nxt, through registers: loaded in one iteration, written to LDS in the
-// next, so each wait is for loads one iteration old.  Block i is rows 16j ..
-// 16j+15, j = min(j0 + jstep * i, jmax); lane 4r+q copies row min(16j + r,
-// last) of src (which points at the lane's four columns) to nxt + 1024 j +
-// 16 lane.  The loads are unconditional (clamped), so no branch splits the
-// load queue; d counts the blocks issued.
-template <bool FAST, bool MORE, int DPI>
+// already loaded.  xb is the lane's view of the chunk's X rows.
+template <bool FAST>
 __device__ __forceinline__ void sell_walk(const int4* __restrict__ blk, int p, int T, const char* __restrict__ xb,
-                                          float4* __restrict__ nxt, const float* __restrict__ src, int64_t ldx,
-                                          int lane, int j0, int jstep, int jmax, int last, int& d, float& a0,
-                                          float& a1, float& a2, float& a3) {
+                                          float& a0, float& a1, float& a2, float& a3) {
     auto comp = [&](const int4 w) {
         float4 xv[8];
         static_for<0, 8>([&](auto tc) {
@@ -1753,25 +1758,7 @@ __device__ __forceinline__ void sell_walk(const int4* __restrict__ blk, int p, i
             }
         }
     };
-    const int r = lane >> 2;
-    constexpr int ND = MORE ? DPI : 1;
-    using f4 = float __attribute__((ext_vector_type(4)));  // a plain vector: stays in registers
-    f4 st[ND];
-    int js[ND];
-    auto load_next = [&]() {
-#pragma unroll
-        for (int i = 0; i < ND; ++i) {
-            js[i] = min(j0 + jstep * (d + i), jmax);
-            st[i] = *reinterpret_cast<const f4*>(src + (int64_t)min(js[i] * 16 + r, last) * ldx);
-        }
-        d += ND;
-    };
-    auto store_next = [&]() {
-#pragma unroll
-        for (int i = 0; i < ND; ++i) *reinterpret_cast<f4*>(nxt + js[i] * 64 + lane) = st[i];
-    };
     int4 w0 = blk[p], w1 = blk[p + 64], w2 = blk[p + 128], w3 = blk[p + 192];
-    if constexpr (MORE) load_next();
     int t = 0;
     for (; t + 4 <= T; t += 4) {
         comp(w0);
@@ -1780,10 +1767,6 @@ __device__ __forceinline__ void sell_walk(const int4* __restrict__ blk, int p, i
         comp(w1);
         w1 = blk[p + 320];
         asm volatile("" ::: "memory");
-        if constexpr (MORE) {
-            store_next();
-            load_next();
-        }
         comp(w2);
         w2 = blk[p + 384];
         asm volatile("" ::: "memory");
@@ -1795,7 +1778,6 @@ __device__ __forceinline__ void sell_walk(const int4* __restrict__ blk, int p, i
     if (t < T) comp(w0);
     if (t + 1 < T) comp(w1);
     if (t + 2 < T) comp(w2);
-    if constexpr (MORE) store_next();
 }
 
 // The walk of one run for the 4-wave launch's walking waves (one wave per
@@ -1916,17 +1898,24 @@ constexpr int sell_threads() { return 64 * (W + (sell_stager<XVEC, W, XT>() ? 1 
 // Gemm multiplies), so no transposed copy is written first.  The 12- and
 // 16-wave launches stage every chunk with all their waves; the 4- and 8-wave launches
 // take it only for one chunk, staged by all their waves.
-template <bool FAST, bool XVEC, int W, bool XT>
+// NF (with XT): the kernel also applies the dense kernels' rule for
+// non-finite activations (k_nonfinite_fix states it).  Every staged value
+// passes a register here, so y * 0 summed per thread tells whether the
+// slice holds one, a wave's verdict waits in LDS for the chunk barrier, and only
+// then does each wave look for the places in its 16 rows.  The separate pass
+// this replaces read X again at one workgroup per 64 x 64: two of the seven
+// device steps of a two-layer network (784-512-10, batch 32: 72 -> 62.5 us).
+template <bool FAST, bool XVEC, int W, bool XT, bool NF>
 __global__ __launch_bounds__((sell_threads<XVEC, W, XT>())) void k_spmm_sell(
     int N, int K, int kc, int nch, int nslab, const int32_t* __restrict__ perm,
     const int32_t* __restrict__ soff, const int4* __restrict__ blk, const float* __restrict__ X,
     int64_t ldx, int nx, float* __restrict__ Y, int64_t ldy_r, int64_t ldy_c, int yvec,
-    const float* __restrict__ bias, int64_t c_size, float beta, int act, float alpha, int scale) {
+    const float* __restrict__ bias, int64_t c_size, float beta, int act, float alpha, int scale,
+    const uint64_t* __restrict__ bm, int64_t nw) {
     // two buffers of kc + 1 rows of 16 floats; row kc of each is zero
     extern __shared__ float4 xs[];
     constexpr int NT = 64 * W;  // the walking waves' threads
     constexpr bool STAGER = sell_stager<XVEC, W, XT>();
-    constexpr int DPI = sell_loads_per_iter<W>();
     const int tid = threadIdx.x, lane = tid & 63, r = lane >> 2, q = lane & 3;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int slab = __builtin_amdgcn_readfirstlane((int)blockIdx.x * W + wave);
@@ -1971,6 +1960,8 @@ __global__ __launch_bounds__((sell_threads<XVEC, W, XT>())) void k_spmm_sell(
     // four groups of 16 lanes in one write instruction hit four different
     // 16-bank quarters (rows 64 B apart would otherwise all meet in one).
     // Rows past N or K are zero.
+    __shared__ int odd_l[W + 1];  // NF: the wave staged a non-finite value
+    float chk = 0.0f;             // NaN once this thread has
     auto stage_xt = [&](int c, int t, int nthr) {
         const int k0 = c * kc, total = 4 * kc;  // 16 rows x kc / 4 pieces
         float* xb = reinterpret_cast<float*>(xs + (c & 1) * bufq);
@@ -1980,6 +1971,14 @@ __global__ __launch_bounds__((sell_threads<XVEC, W, XT>())) void k_spmm_sell(
             for (int i = 0; i < 8; ++i) {
                 const int e = min(e0 + t + nthr * i, total - 1), n = e & 15, k = k0 + 4 * (e >> 4);
                 v[i] = *reinterpret_cast<const float4*>(X + (int64_t)min(n0 + n, N - 1) * ldx + min(k, K - 4));
+            }
+            if constexpr (NF) {
+#pragma unroll
+                for (int i = 0; i < 8; ++i) {  // a clamped piece is another of the slice
+                    const float a[4] = {v[i].x, v[i].y, v[i].z, v[i].w};
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) chk = __builtin_fmaf(scale ? alpha * a[j] : a[j], 0.0f, chk);
+                }
             }
 #pragma unroll
             for (int i = 0; i < 8; ++i) {
@@ -1997,6 +1996,10 @@ __global__ __launch_bounds__((sell_threads<XVEC, W, XT>())) void k_spmm_sell(
                     }
                 }
             }
+        }
+        if constexpr (NF) {
+            const uint64_t odd = __ballot(chk != chk);
+            if (lane == 0) odd_l[wave] = odd != 0;
         }
     };
     auto sync_chunk = [&]() {
@@ -2035,15 +2038,13 @@ __global__ __launch_bounds__((sell_threads<XVEC, W, XT>())) void k_spmm_sell(
         __syncthreads();
         for (int c = 0; c < nch; ++c) {
             const char* xb = reinterpret_cast<const char*>(xs + (c & 1) * bufq) + q * 16;
-            int d = 0;
             if (slab < nslab) {
                 const int s0 = soff[slab * (nch + 1) + c], s1 = soff[slab * (nch + 1) + c + 1];
                 const int T = __builtin_amdgcn_readfirstlane((s1 - s0) / 64);
                 if constexpr (W == 4)
                     sell_walk_pipe<FAST>(blk, s0 + lane, T, xb, a0, a1, a2, a3);
                 else
-                    sell_walk<FAST, false, DPI>(blk, s0 + lane, T, xb, xs, xcol, ldx, lane, wave, W, nld - 1, 0, d,
-                                                a0, a1, a2, a3);
+                    sell_walk<FAST>(blk, s0 + lane, T, xb, a0, a1, a2, a3);
             }
             if (c + 1 < nch) __syncthreads();
         }
@@ -2058,31 +2059,20 @@ __global__ __launch_bounds__((sell_threads<XVEC, W, XT>())) void k_spmm_sell(
     sync_chunk();
     for (int c = 0; c < nch; ++c) {
         const char* xb = reinterpret_cast<const char*>(xs + (c & 1) * bufq) + q * 16;
-        int d = 0;  // loads of chunk c + 1 issued by this wave
         const bool more = c + 1 < nch;
         if (slab < nslab) {
             const int s0 = soff[slab * (nch + 1) + c], s1 = soff[slab * (nch + 1) + c + 1];
             const int T = __builtin_amdgcn_readfirstlane((s1 - s0) / 64);
-            const int k1 = (c + 1) * kc;
-            float4* nxt = xs + ((c + 1) & 1) * bufq;
-            // the 16-wave launch (four waves per SIMD hide each other's
-            // latencies) stages whole chunks between walks instead
-            if constexpr (W == 4)
-                sell_walk_pipe<FAST>(blk, s0 + lane, T, xb, a0, a1, a2, a3);
-            else if (XVEC && !XT && W <= 8 && more)
-                sell_walk<FAST, true, DPI>(blk, s0 + lane, T, xb, nxt, xcol + (int64_t)k1 * ldx, ldx, lane, wave, W,
-                                           nld - 1, min(kc, K - k1) - 1, d, a0, a1, a2, a3);
-            else
-                sell_walk<FAST, false, DPI>(blk, s0 + lane, T, xb, nxt, xcol, ldx, lane, wave, W, nld - 1, 0, d, a0,
-                                            a1, a2, a3);
+            if constexpr (W == 4) sell_walk_pipe<FAST>(blk, s0 + lane, T, xb, a0, a1, a2, a3);
+            else sell_walk<FAST>(blk, s0 + lane, T, xb, a0, a1, a2, a3);
         }
         if (more) {
             if constexpr (XT) {
                 stage_xt(c + 1, tid, NT);  // the other buffer: last read in chunk c - 1
             } else if constexpr (XVEC) {
-                for (; d < nd; ++d) dma(c + 1, d);
+                for (int i = 0; i < nd; ++i) dma(c + 1, i);  // the other buffer: last read in chunk c - 1
             } else {
-                for (int i = 0; i < nd1; ++i) dma1(c + 1, i);  // the other buffer: last read in chunk c - 1
+                for (int i = 0; i < nd1; ++i) dma1(c + 1, i);
             }
             sync_chunk();
         }
@@ -2091,6 +2081,18 @@ __global__ __launch_bounds__((sell_threads<XVEC, W, XT>())) void k_spmm_sell(
     if (slab < nslab) {
         const int row = perm[slab * pfr::kSellRows + r];
         const int cn = n0 + q * 4;
+        if constexpr (NF) {
+            int odd = 0;
+            for (int i = 0; i < (STAGER ? W + 1 : W); ++i) odd |= odd_l[i];
+            if (__builtin_amdgcn_readfirstlane(odd) != 0) {
+                const int hit = sell_nonfinite(X, ldx, n0, N, K, alpha, scale, bm, nw, row, q);
+                const float qnan = __builtin_nanf("");
+                if (hit & 1) a0 = qnan;
+                if (hit & 2) a1 = qnan;
+                if (hit & 4) a2 = qnan;
+                if (hit & 8) a3 = qnan;
+            }
+        }
         if (row >= 0 && cn < N) {
             float* yr = Y + (int64_t)row * ldy_r;
             if (yvec && cn + 3 < N) {
@@ -2138,11 +2140,11 @@ const int4* sell_runs(const pfr_csr* W, bool fast) {
 }
 
 // Column-slice kernel launch with W waves per workgroup.
-template <bool FAST, bool XVEC, int W, bool XT>
+template <bool FAST, bool XVEC, int W, bool XT, bool NF>
 void launch_sell_w(pfr_ctx* ctx, const pfr_csr* Wt, const float* X, int N, int64_t ldx, int nx, float* Y,
                    int64_t ldy_r, int64_t ldy_c, int yvec, const float* bias, int64_t c_size, float beta, int act,
                    float alpha) {
-    auto kern = k_spmm_sell<FAST, XVEC, W, XT>;
+    auto kern = k_spmm_sell<FAST, XVEC, W, XT, NF>;
     const size_t lds = (size_t)(Wt->sell_kc + 1) * 64 * (Wt->sell_nch > 1 ? 2 : 1);
     // more than 64 KiB of dynamic LDS has to be allowed per kernel and device
     static uint64_t allowed = 0;  // bit d: done on device d (< 64)
@@ -2155,7 +2157,8 @@ void launch_sell_w(pfr_ctx* ctx, const pfr_csr* Wt, const float* X, int N, int64
     dim3 grid((unsigned)((Wt->sell_nslab + W - 1) / W), (unsigned)((N + pfr::kSellCols - 1) / pfr::kSellCols));
     hipLaunchKernelGGL(kern, grid, dim3(sell_threads<XVEC, W, XT>()), lds, ctx->stream, N, (int)Wt->K,
                        Wt->sell_kc, Wt->sell_nch, Wt->sell_nslab, Wt->sell_perm, Wt->sell_soff, sell_runs(Wt, FAST), X, ldx,
-                       nx, Y, ldy_r, ldy_c, yvec, bias, c_size, beta, act, alpha, alpha != 1.0f ? 1 : 0);
+                       nx, Y, ldy_r, ldy_c, yvec, bias, c_size, beta, act, alpha, alpha != 1.0f ? 1 : 0,
+                       Wt->pattern, Wt->pattern_nw);
 }
 
 // Waves per workgroup of the column-slice launch for N columns, and its
@@ -2179,12 +2182,12 @@ int sell_waves(const pfr_ctx* ctx, const pfr_csr* Wt, int64_t N, int64_t* rounds
     return w;
 }
 
-template <bool FAST, bool XVEC, bool XT>
+template <bool FAST, bool XVEC, bool XT, bool NF = false>
 void launch_sell_x(pfr_ctx* ctx, const pfr_csr* Wt, const float* X, int N, int64_t ldx, int nx, float* Y,
                    int64_t ldy_r, int64_t ldy_c, int yvec, const float* bias, int64_t c_size, float beta, int act,
                    float alpha) {
 #define PFR_SELLW(WV) \
-    launch_sell_w<FAST, XVEC, WV, XT>(ctx, Wt, X, N, ldx, nx, Y, ldy_r, ldy_c, yvec, bias, c_size, beta, act, alpha)
+    launch_sell_w<FAST, XVEC, WV, XT, NF>(ctx, Wt, X, N, ldx, nx, Y, ldy_r, ldy_c, yvec, bias, c_size, beta, act, alpha)
     const int w = sell_waves(ctx, Wt, N);
     if (w == 16) PFR_SELLW(16);
     else if (w == 12) PFR_SELLW(12);
@@ -2201,10 +2204,13 @@ void launch_sell(pfr_ctx* ctx, const pfr_csr* Wt, const float* X, int N, int64_t
     const int nx = padded ? (N + 3) / 4 * 4 : N;
     const bool xvec = (ldx % 4 == 0) && (nx % 4 == 0) && aligned16(X);
     const int yvec = (ldy_c == 1 && ldy_r % 4 == 0 && aligned16(Y) && bias == nullptr) ? 1 : 0;
-#define PFR_SELLX(F, XV, T) \
-    launch_sell_x<F, XV, T>(ctx, Wt, X, N, ldx, nx, Y, ldy_r, ldy_c, yvec, bias, c_size, beta, act, alpha)
+#define PFR_SELLX(F, XV, ...) \
+    launch_sell_x<F, XV, __VA_ARGS__>(ctx, Wt, X, N, ldx, nx, Y, ldy_r, ldy_c, yvec, bias, c_size, beta, act, alpha)
     if (xt) {
-        if (fast) PFR_SELLX(true, false, true);
+        const bool nf = Wt->pattern != nullptr;
+        if (fast && nf) PFR_SELLX(true, false, true, true);
+        else if (fast) PFR_SELLX(true, false, true);
+        else if (nf) PFR_SELLX(false, false, true, true);
         else PFR_SELLX(false, false, true);
     } else if (fast) {
         if (xvec) PFR_SELLX(true, true, false);
@@ -2341,11 +2347,10 @@ void launch_csr_kernels(pfr_ctx* ctx, const pfr_csr* W, const float* X, int64_t 
 // and an inf mask (ballots), and only a column with either walks the rows,
 // writing the epilogue of NaN (bias and activation as the product kernels
 // apply them) where the rule says so.  Columns without non-finite values --
-// the normal case -- cost one read of X.  x[k, c] is X[k * sk + c * sn]
-// (sn = 1: X as the products read it; sk = 1: the Gemm form's activation
-// read in place), times alpha when `scale`.
-__global__ __launch_bounds__(256) void k_nonfinite_fix(const float* __restrict__ X, int64_t sk, int64_t sn,
-                                                       float alpha, int scale, int64_t K, int64_t N, int64_t M,
+// the normal case -- cost one read of X.  (A column-slice launch that reads
+// the Gemm form's activation in place applies the rule itself.)
+__global__ __launch_bounds__(256) void k_nonfinite_fix(const float* __restrict__ X, int64_t ldx, int64_t K,
+                                                       int64_t N, int64_t M,
                                                        const uint64_t* __restrict__ bm, int64_t nw,
                                                        float* __restrict__ Y, int64_t ldy_r, int64_t ldy_c,
                                                        const float* __restrict__ bias, int64_t c_size, float beta,
@@ -2353,11 +2358,9 @@ __global__ __launch_bounds__(256) void k_nonfinite_fix(const float* __restrict__
     __shared__ float t[64][65];  // t[c][k]
     const int64_t kt = blockIdx.x, k0 = kt * 64, c0 = (int64_t)blockIdx.y * 64;
     for (int e = threadIdx.x; e < 64 * 64; e += 256) {
-        // consecutive threads along whichever index X's rows run
-        const int cc = sn == 1 ? e % 64 : e / 64, kk = sn == 1 ? e / 64 : e % 64;
+        const int cc = e % 64, kk = e / 64;
         const int64_t k = k0 + kk, c = c0 + cc;
-        const float v = (k < K && c < N) ? X[k * sk + c * sn] : 0.0f;
-        t[cc][kk] = scale ? alpha * v : v;
+        t[cc][kk] = (k < K && c < N) ? X[k * ldx + c] : 0.0f;
     }
     __syncthreads();
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -2414,12 +2417,11 @@ void launch_spmm(pfr_ctx* ctx, const pfr_csr* W, const float* X, int64_t N, int6
         else launch_csr_kernels<false, false>(ctx, W, X, N, ldx, Y, ldy_r, ldy_c, bias, c_size, beta, act);
     }
     PFR_HIP(hipGetLastError());
-    if (W->pattern != nullptr && W->K > 0) {
+    if (W->pattern != nullptr && W->K > 0 && !xt) {  // the column-slice kernel does it with xt
         pfr::require((N + 63) / 64 < 65536, "too many columns for the non-finite fix-up's grid");
         const dim3 grid((unsigned)((W->K + 63) / 64), (unsigned)((N + 63) / 64));
-        hipLaunchKernelGGL(k_nonfinite_fix, grid, dim3(256), 0, ctx->stream, X, xt ? (int64_t)1 : ldx,
-                           xt ? ldx : (int64_t)1, alpha, xt && alpha != 1.0f ? 1 : 0, W->K, N, W->M, W->pattern,
-                           W->pattern_nw, Y, ldy_r, ldy_c, bias, c_size, beta, act);
+        hipLaunchKernelGGL(k_nonfinite_fix, grid, dim3(256), 0, ctx->stream, X, ldx,
+                           W->K, N, W->M, W->pattern, W->pattern_nw, Y, ldy_r, ldy_c, bias, c_size, beta, act);
         PFR_HIP(hipGetLastError());
     }
 }

@@ -65,3 +65,51 @@ def test_widths(ctx, M, K, widths):
             g = terms * 2.0 ** -24
             assert (np.abs(F - exact) <= g / (1 - g) * mag + 1e-30).all()
         W.free()
+
+
+@pytest.mark.parametrize("M,K,N,alpha,act", [
+    (16, 64, 9, 1.0, None),       # one slab, one chunk
+    (500, 784, 32, 1.0, "relu"),  # one chunk, a staging wave
+    (515, 1020, 33, -2.0, None),  # alpha applied before the test for infinities
+    (515, 2052, 47, 1.0, "gelu"),
+    (3100, 1500, 200, 1.0, None),  # two chunks, 12 waves
+    (4096, 2000, 256, 1.0, None)])  # two chunks, 16 waves
+def test_nonfinite_rule_in_kernel(ctx, M, K, N, alpha, act):
+    """A handle with the dense kernels' semantics, Gemm form: the launch that
+    stages the activation itself makes exactly the outputs NaN that cpu_gemm
+    on the zero-filled weight does, as do the launches after a transpose."""
+    import torch
+
+    rng = np.random.default_rng(M + K + N)
+    ip, ix, v = workloads.csr_uniform(M, K, 0.06, 0.05, seed=M + N)
+    W = ctx.csr_upload(M, K, ip, ix, v)
+    W.dense_semantics()
+    Wt = np.ascontiguousarray(workloads.csr_to_dense(M, K, ip, ix, v).T)
+    b = workloads.dense_normal((M,), 0.1, seed=M)
+    A = workloads.dense_normal((N, K), 1.0, seed=N)
+    A[0, K - 1], A[N // 2, 0], A[N - 1, K // 2] = np.inf, np.nan, -np.inf
+    if alpha != 1.0:
+        A[2, 3] = 3e38  # infinite once scaled
+    db, dA = torch.from_numpy(b).cuda(), torch.from_numpy(A).cuda()
+    dY = torch.empty((N, M), device="cuda")
+    for bad in (True, False):
+        if not bad:  # and finite activations leave every bit alone
+            A = np.where(np.abs(A) < 100, A, 0).astype(np.float32)
+            dA = torch.from_numpy(A).cuda()
+        print(f"non-finite rule M={M} K={K} N={N} bad={bad}", flush=True)
+        torch.cuda.synchronize()
+        W_args = dict(relu=act == "relu", gelu=act == "gelu")
+        ctx.gemm_csr_dev(dA.data_ptr(), N, K, W, dY.data_ptr(), alpha, 1.0, db.data_ptr(), M, mode="strict", **W_args)
+        ctx.synchronize()
+        Y = dY.cpu().numpy()
+        with np.errstate(all="ignore"):
+            R = O.orc_gemm(A, Wt, b, alpha, 1.0, 0, 0)
+        if act == "relu":
+            R = np.where(0 < R, R, 0).astype(np.float32)
+        if act == "gelu":
+            assert np.array_equal(np.isnan(Y), np.isnan(ctx.gelu(R)))
+            continue
+        assert np.array_equal(np.isnan(Y), np.isnan(R))
+        ok = ~np.isnan(R)
+        assert np.array_equal(Y[ok].view(np.uint32), R[ok].view(np.uint32))
+    W.free()
