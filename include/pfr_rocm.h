@@ -57,7 +57,7 @@ typedef enum pfr_act {
     PFR_ACT_NONE = 0,
     PFR_ACT_RELU = 1, /* cpu_relu, activation.cpp:45-60: std::max(0.0f, v) */
     PFR_ACT_GELU = 2  /* cpu_gelu, activation.cpp:239-259: tanh approximation
-                         (device tanhf: within a few ulp of the reference) */
+                         (as v / (1 + exp(-2u)): within a few ulp of the reference) */
 } pfr_act;
 
 typedef struct pfr_ctx pfr_ctx;   /* one device + one stream + scratch */
@@ -152,7 +152,8 @@ int pfr_csr_info(const pfr_csr* w, int64_t* M, int64_t* K, int64_t* nnz);
 /* Device bytes the handle holds: the CSR itself (row pointers, columns as
  * uint16 when K <= 65536 and int32 otherwise, values, row scales), the
  * row-block table, the merge-path partition and every derived copy built so
- * far.  The sliced-ELL copy (float32 weights, N >= 16; one in storage order
+ * far.  The sliced-ELL copy (N >= 9; int8 weights hold their dequantised
+ * float32 values in it, 8 bytes a step; one in storage order
  * for the strict mode, one reordered for the fast mode, sharing their slab
  * tables), the row-chain copy (strict, N <= 8) and the nnz-balanced copy
  * (fast, N <= 8) are built by the
@@ -351,7 +352,7 @@ int pfr_softmax(pfr_ctx* ctx, const float* x, int64_t outer, int64_t axis,
 int pfr_softmax_dev(pfr_ctx* ctx, const float* x, int64_t outer, int64_t axis,
                     int64_t inner, float* y);
 /* Gelu, cpu_gelu (activation.cpp:239-259): 0.5 x (1 + tanh(sqrt(2/pi)
- * (x + 0.044715 x^3))) with the device tanhf (a few ulp from the CPU). */
+ * (x + 0.044715 x^3))) as x / (1 + exp(-2u)) (a few ulp from the CPU). */
 int pfr_gelu(pfr_ctx* ctx, const float* x, int64_t n, float* y);
 int pfr_gelu_dev(pfr_ctx* ctx, const float* x, int64_t n, float* y);
 /* Add with numpy broadcasting (cpu_add, math.cpp:150-224), bit-exact; at

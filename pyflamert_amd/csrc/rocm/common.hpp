@@ -166,9 +166,8 @@ struct pfr_csr {
     int32_t max_row_nnz = 0;
     // Columns ascend within every row (the order to_sparse produces).
     bool cols_sorted = false;
-    // Sliced-ELL copy for the column-slice kernel (float32 steps, also for int8
-    // values; null
-    // when the shape does not qualify).  Rows are reordered into slabs of
+    // Sliced-ELL copy for the column-slice kernel (float32 steps, for int8 values
+    // too; null when the shape does not qualify).  Rows are reordered into slabs of
     // kSellRows; K is cut into chunks of sell_kc rows (a multiple of 16, at
     // most kSellMaxKC; the last chunk may be partial).  For slab s and chunk
     // c, sell_soff[s * (sell_nch + 1) + c] is the first int4 of its run of
