@@ -1872,8 +1872,9 @@ __device__ __forceinline__ void sell_walk_pipe(const int4* __restrict__ blk, int
 // load per wave instruction), by a staging wave beside the walk or by each
 // wave that has finished its own.  (Issued ahead of the walk, with the LDS
 // reads kept from waiting for them, N = 256 took 38.1 - 39.0 us against 37.7:
-// the copies queue in front of the weight loads.)  Each wave walks its slab: lane 4r+q accumulates columns 4q..4q+3 of slab row r.  The pairs of a
-// step come from one int4 per lane per eight steps, broadcast to the row's
+// the copies queue in front of the weight loads.)  Each wave walks its slab:
+// lane 4r+q accumulates columns 4q..4q+3 of slab row r.  The pairs of a step
+// come from one int4 per lane per eight steps, broadcast to the row's
 // four lanes with quad_perm DPP (which the compiler folds into the address
 // add and the multiply).  Products are added in the row's storage order, so
 // strict mode matches the row kernels bit for bit; padding steps add
