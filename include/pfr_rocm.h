@@ -57,7 +57,7 @@ typedef enum pfr_act {
     PFR_ACT_NONE = 0,
     PFR_ACT_RELU = 1, /* cpu_relu, activation.cpp:45-60: std::max(0.0f, v) */
     PFR_ACT_GELU = 2  /* cpu_gelu, activation.cpp:239-259: tanh approximation
-                         (as v / (1 + exp(-2u)): within a few ulp of the reference) */
+                         (the bits and the bound of pfr_gelu) */
 } pfr_act;
 
 typedef struct pfr_ctx pfr_ctx;   /* one device + one stream + scratch */
@@ -352,7 +352,10 @@ int pfr_softmax(pfr_ctx* ctx, const float* x, int64_t outer, int64_t axis,
 int pfr_softmax_dev(pfr_ctx* ctx, const float* x, int64_t outer, int64_t axis,
                     int64_t inner, float* y);
 /* Gelu, cpu_gelu (activation.cpp:239-259): 0.5 x (1 + tanh(sqrt(2/pi)
- * (x + 0.044715 x^3))) as x / (1 + exp(-2u)) (a few ulp from the CPU). */
+ * (x + 0.044715 x^3))) as x / (1 + exp(-2u)), u the argument of tanh:
+ * within 2.4e-7 |x| + 1e-6 |y| of the CPU's y (whose 1 + tanhf(u) cancels for
+ * negative x, so ulps of y are no measure there), NaN, infinities and signed
+ * zeros alike. */
 int pfr_gelu(pfr_ctx* ctx, const float* x, int64_t n, float* y);
 int pfr_gelu_dev(pfr_ctx* ctx, const float* x, int64_t n, float* y);
 /* Add with numpy broadcasting (cpu_add, math.cpp:150-224), bit-exact; at

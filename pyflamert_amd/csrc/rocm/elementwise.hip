@@ -6,7 +6,7 @@
 //              divide; all -inf (or zero sum) rows become uniform 1/n.  exp
 //              is the device expf, so results match the CPU within a few
 //              ulp, not bit for bit.
-//   Gelu       activation.cpp:239-259 (pfr::gelu, a few ulp).
+//   Gelu       activation.cpp:239-259 (pfr::gelu, within 2.4e-7 |x| + 1e-6 |y|).
 //   Add        math.cpp:150-224: numpy-style broadcasting, bit-exact.
 //   LayerNorm  nn.cpp:419-490: per row a sequential mean and variance in one
 //              thread (the reference's summation order), then

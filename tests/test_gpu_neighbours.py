@@ -4,10 +4,10 @@ on the device-resident plan.
 
 Bars: Add and LayerNormalization bit-exact against the golden vectors
 written by the compiled reference and against the oracle; Gelu within
-|d| <= 2.4e-7 * |x| + 1e-6 * |y| of the reference (the device tanhf against
-glibc's: a few ulp of tanh, which 0.5 * x * (1 + tanh) carries as an absolute
-error proportional to |x| where 1 + tanh cancels), the special values (NaN,
-+-inf, signed zero) identical.  Fusing Gelu into the product's epilogue
+|d| <= 2.4e-7 * |x| + 1e-6 * |y| of the reference (an ulp of its tanhf, which
+0.5 * x * (1 + tanh) carries as an absolute error proportional to |x| where 1 +
+tanh cancels) and no further from 64 bits than the reference itself, the
+special values (NaN, +-inf, signed zero) identical.  Fusing Gelu into the product's epilogue
 changes no bit.
 """
 import sys
@@ -68,6 +68,26 @@ def test_gelu(ctx, golden):
     say("Gelu: 1M N(0, 16) values against the oracle")
     gelu_close(x, ctx.gelu(x), O.orc_gelu(x))
     assert ctx.gelu(np.zeros(0, np.float32)).size == 0
+
+
+def test_gelu_error(ctx):
+    """Against the same function in 64 bits, interval by interval: the GPU's
+    error (2-norm) is no larger than that of the reference's float32 sequence
+    with a correctly rounded tanh, which leaves out its own tanhf's error."""
+    rng = np.random.default_rng(8)
+    for lo, hi in ((-5, -3), (-3, -2), (-2, -1), (-1, -0.5), (-0.5, -0.1), (-0.1, 0), (0, 0.1), (0.1, 0.5), (0.5, 1),
+                   (1, 2), (2, 3), (3, 5)):
+        x = rng.uniform(lo, hi, 1 << 18).astype(np.float32)
+        u = np.float32(0.7978845608028654) * (x + np.float32(0.044715) * x * x * x)
+        ref = np.float32(0.5) * x * (np.float32(1) + np.tanh(u.astype(np.float64)).astype(np.float32))
+        x64 = x.astype(np.float64)
+        exact = x64 / (1 + np.exp(-2 * np.sqrt(2 / np.pi) * (x64 + 0.044715 * x64 ** 3)))
+        got, of_ref = (np.linalg.norm(y.astype(np.float64) - exact) / np.linalg.norm(exact) for y in (ctx.gelu(x), ref))
+        say(f"Gelu on [{lo}, {hi}]: error {got:.3g}, the reference's sequence {of_ref:.3g}")
+        assert got <= of_ref
+    x = np.array([0.0, -0.0, 1e-40, -1e-40, 1e38, -1e38, np.inf, -np.inf, np.nan], np.float32)
+    with np.errstate(all="ignore"):
+        assert same(np.nan_to_num(ctx.gelu(x), nan=7.0), np.nan_to_num(O.orc_gelu(x), nan=7.0))
 
 
 def test_add(ctx, golden):
