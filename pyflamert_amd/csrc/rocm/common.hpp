@@ -311,6 +311,10 @@ namespace pfr {
 void bind(pfr_ctx* ctx);
 // Derived copies of a CSR weight, built on first use.
 constexpr uint32_t kCopySell = 1, kCopyChain = 2, kCopyBal = 4, kCopySellFast = 8;
+// Whether w's copy of this bit may be looked at: a build clears the bit last.  A
+// product that does not wait for another thread's build (the allocation-free
+// entry) finds the pointers of a copy half made without asking.
+inline bool copy_settled(const pfr_csr* w, uint32_t bit) { return (w->pending.load(std::memory_order_acquire) & bit) == 0; }
 // Builds the copies among `which` that w still has pending, on w's context
 // stream (allocates, plans on the host and fills on the device, then
 // synchronizes).  A copy whose plan does not fit is dropped from pending and

@@ -2141,7 +2141,8 @@ int next_pow2(int n) {
 
 // The sliced-ELL runs a product in this mode reads (null: neither copy).
 const int4* sell_runs(const pfr_csr* W, bool fast) {
-    return fast && W->sell_blk_fast != nullptr ? W->sell_blk_fast : W->sell_blk;
+    if (fast && pfr::copy_settled(W, pfr::kCopySellFast) && W->sell_blk_fast != nullptr) return W->sell_blk_fast;
+    return pfr::copy_settled(W, pfr::kCopySell) ? W->sell_blk : nullptr;
 }
 
 // Column-slice kernel launch with W waves per workgroup.
@@ -2280,11 +2281,13 @@ void launch_csr_kernels(pfr_ctx* ctx, const pfr_csr* W, const float* X, int64_t 
     hipStream_t s = ctx->stream;
     const void* val = W->val;
     const float* rs = W->row_scale;
+    const bool bal = FAST && pfr::copy_settled(W, pfr::kCopyBal) && W->bal_meta != nullptr;
+    const bool chain = !FAST && pfr::copy_settled(W, pfr::kCopyChain) && W->chain_q0 != nullptr;
     if (FAST && N == 1 && ctx->merge && W->mp_wave != nullptr && ldx < INT32_MAX) {
         launch_merge<I8>(ctx, W, X, ldx, Y, ldy_r, bias, c_size, beta, act);
-    } else if (FAST && N == 1 && W->bal_meta != nullptr && ldx < INT32_MAX) {
+    } else if (bal && N == 1 && ldx < INT32_MAX) {
         launch_bal_fast<I8>(ctx, W, X, ldx, Y, ldy_r, bias, c_size, beta, act);
-    } else if (FAST && N >= 2 && N <= 8 && W->bal_meta != nullptr) {
+    } else if (bal && N >= 2 && N <= 8) {
         if (N == 8 && ldx % 4 == 0 && aligned16(X))
             launch_bal_fast8<I8, true>(ctx, W, X, (int)N, ldx, Y, ldy_r, ldy_c, bias, c_size, beta, act);
         else
@@ -2320,13 +2323,13 @@ void launch_csr_kernels(pfr_ctx* ctx, const pfr_csr* W, const float* X, int64_t 
         }
 #undef PFR_FASTC
 #undef PFR_FASTV
-    } else if (N == 1 && W->chain_q0 != nullptr && W->chain_xlds && ldx < INT32_MAX) {
+    } else if (chain && N == 1 && W->chain_xlds && ldx < INT32_MAX) {
         if (W->chain_rows == 16) launch_chain_x<I8, 16>(ctx, W, X, ldx, Y, ldy_r, bias, c_size, beta, act);
         else if (W->chain_rows == 32) launch_chain_x<I8, 32>(ctx, W, X, ldx, Y, ldy_r, bias, c_size, beta, act);
         else launch_chain_x<I8, 64>(ctx, W, X, ldx, Y, ldy_r, bias, c_size, beta, act);
-    } else if (N >= 2 && N <= 8 && W->chain_q0 != nullptr && W->chain_rows % kChainNR == 0 && W->chain_c16) {
+    } else if (chain && N >= 2 && N <= 8 && W->chain_rows % kChainNR == 0 && W->chain_c16) {
         launch_chain_cols<I8>(ctx, W, X, (int)N, ldx, Y, ldy_r, ldy_c, bias, c_size, beta, act);
-    } else if (N == 1 && W->chain_q0 != nullptr && W->K * ldx < INT32_MAX) {
+    } else if (chain && N == 1 && W->K * ldx < INT32_MAX) {
         const dim3 grid((unsigned)W->chain_nslab), block(64 * (kChainP + 1));
         if (W->chain_c16)
             hipLaunchKernelGGL((k_spmv_chain<I8, true>), grid, block, 0, s, W->chain_q0, W->chain_len,

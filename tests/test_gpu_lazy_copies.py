@@ -168,3 +168,60 @@ def test_capture_before_copy_reads_in_place(ctx):
         assert close_normwise(out["f8"].cpu().numpy(), R["f8"]), rep
     del graph
     W.free()
+
+
+@pytest.mark.parametrize("values", ["f32", "i8"])
+@pytest.mark.parametrize("Mb", [4, 32])
+def test_allocation_free_products_beside_a_build(ctx, values, Mb):
+    """One thread's allocation-free products on its own stream, which wait for
+    no build, while another thread's first products through the same handle
+    build the row-chain, balanced and both sliced-ELL copies: each result is
+    the oracle's, bit for bit, whether it read the CSR in place or a copy that
+    was complete."""
+    import threading
+
+    import torch
+
+    from pyflamert_amd import rocm
+
+    M, K = 4096, 1536
+    ip, ix, q, sc = workloads.csr_int8_lognormal(M, K, 0.2, 0.5, 0.02, seed=45)
+    vals = workloads.dequant_rows(ip, q, sc)
+    A = workloads.dense_normal((Mb, K), 1.0, seed=46)
+    X = np.ascontiguousarray(A.T)
+    R = O.orc_csr_spmm(M, K, ip, ix, vals, X).T
+    other = rocm.Context(0)
+    dA = torch.from_numpy(A).cuda()
+    dY = torch.empty((Mb, M), device="cuda")
+    torch.cuda.synchronize()
+    for rep in range(4):
+        W = ctx.csr_upload(M, K, ip, ix, vals) if values == "f32" else ctx.csr_upload(M, K, ip, ix, q, row_scales=sc)
+        failed, done = [], threading.Event()
+
+        def build():
+            try:
+                for mode in ("strict", "fast"):
+                    Y = W.spmm(X, mode=mode)
+                    if mode == "strict" and not np.array_equal(bits(Y), bits(R.T)):
+                        failed.append("the building product")
+            except Exception as e:
+                failed.append(repr(e))
+            finally:
+                done.set()
+
+        t = threading.Thread(target=build)
+        t.start()
+        n, last = 0, False
+        while not last:  # once more after the build
+            last = done.is_set()
+            other.gemm_csr_dev(dA.data_ptr(), Mb, K, W, dY.data_ptr(), mode="strict", noalloc=True)
+            other.synchronize()
+            n += 1
+            if not np.array_equal(bits(dY.cpu().numpy()), bits(R)):
+                failed.append(f"allocation-free product {n}")
+                break
+        t.join()
+        say(f"{values} Mb={Mb} build {rep}: {n} allocation-free products beside it")
+        assert not failed, failed
+        W.free()
+    other.close()
