@@ -1381,12 +1381,13 @@ std::vector<int32_t> row_lengths(const pfr_csr* w) {
 }
 
 // Sliced-ELL copy (float32 steps, V the weight's values), planned from the
-// kept chunk counts.
+// kept chunk counts.  The tables go over through st, which the caller keeps
+// until the stream has been synchronized, also when this throws.
 template <class CI, class V>
-void fill_sell(pfr_csr* w, const CI* col, hipStream_t s) {
+void fill_sell(pfr_csr* w, const CI* col, Staging& st, hipStream_t s) {
     SellPlan p;
     if (!plan_sell(w->M, w->K, w->h_sell_cnt, &p)) return;
-    Staging st(w->ctx, sell_table_bytes(p));
+    st = Staging(w->ctx, sell_table_bytes(p));
     w->sell_blk = walloc<int4>(w, p.len + pfr::kSellTail);
     const int32_t pad = (int32_t)(p.kc * 64);
     fill_dev(w->sell_blk, p.len + pfr::kSellTail, make_int4(pad, 0, pad, 0), s);
@@ -1404,10 +1405,10 @@ void fill_sell(pfr_csr* w, const CI* col, hipStream_t s) {
 // storage order when a row repeats columns until a chunk of it holds more
 // entries than the chunk has columns.
 template <class CI, class V>
-void fill_sell_fast(pfr_csr* w, const CI* col, hipStream_t s) {
+void fill_sell_fast(pfr_csr* w, const CI* col, Staging& st, hipStream_t s) {
     SellPlan p;
     if (!plan_sell(w->M, w->K, w->h_sell_cnt, &p)) return;
-    Staging st(w->ctx, sell_table_bytes(p));
+    st = Staging(w->ctx, sell_table_bytes(p));
     w->sell_blk_fast = walloc<int4>(w, p.len + pfr::kSellTail);
     const int32_t pad = (int32_t)(p.kc * 64);
     fill_dev(w->sell_blk_fast, p.len + pfr::kSellTail, make_int4(pad, 0, pad, 0), s);
@@ -1509,10 +1510,10 @@ void fill_bal(pfr_csr* w, const CI* col, hipStream_t s) {
 }
 
 template <class CI>
-void build_copy(pfr_csr* w, uint32_t bit, const CI* col, hipStream_t s) {
+void build_copy(pfr_csr* w, uint32_t bit, const CI* col, Staging& st, hipStream_t s) {
     const bool i8 = w->vdt == PFR_I8;
-    if (bit == pfr::kCopySell) i8 ? fill_sell<CI, int8_t>(w, col, s) : fill_sell<CI, float>(w, col, s);
-    else if (bit == pfr::kCopySellFast) i8 ? fill_sell_fast<CI, int8_t>(w, col, s) : fill_sell_fast<CI, float>(w, col, s);
+    if (bit == pfr::kCopySell) i8 ? fill_sell<CI, int8_t>(w, col, st, s) : fill_sell<CI, float>(w, col, st, s);
+    else if (bit == pfr::kCopySellFast) i8 ? fill_sell_fast<CI, int8_t>(w, col, st, s) : fill_sell_fast<CI, float>(w, col, st, s);
     else if (bit == pfr::kCopyChain) i8 ? fill_chain<CI, int8_t>(w, col, s) : fill_chain<CI, float>(w, col, s);
     else i8 ? fill_bal<CI, int8_t>(w, col, s) : fill_bal<CI, float>(w, col, s);
 }
@@ -1708,9 +1709,10 @@ void csr_build_copies(pfr_csr* w, uint32_t which) {
     for (const uint32_t bit : {kCopySell, kCopySellFast, kCopyChain, kCopyBal}) {
         if ((which & bit) == 0) continue;
         const int64_t before = w->dev_bytes;
+        Staging st;  // outlives the copies from it, a failed build's too
         try {
-            if (w->col16) build_copy(w, bit, w->col16, s);
-            else build_copy(w, bit, w->col, s);
+            if (w->col16) build_copy(w, bit, w->col16, st, s);
+            else build_copy(w, bit, w->col, st, s);
         } catch (...) {
             (void)hipStreamSynchronize(s);
             drop_copy(w, bit);

@@ -225,3 +225,48 @@ def test_allocation_free_products_beside_a_build(ctx, values, Mb):
         assert not failed, failed
         W.free()
     other.close()
+
+
+def test_two_threads_build_on_one_context(ctx):
+    """Two threads building handles, from a host CSR and from a dense device
+    weight, and their sliced-ELL copies on one context at once: one of them has
+    the context's page-locked and counting buffers, the other memory of its
+    own; every product is the oracle's."""
+    import threading
+
+    import torch
+
+    N = 16
+    work = []
+    for i, (M, K) in enumerate(((2048, 1500), (3000, 700))):
+        ip, ix, v = workloads.csr_uniform(M, K, 0.1, 0.02, seed=50 + i)
+        X = workloads.dense_normal((K, N), 1.0, seed=60 + i)
+        work.append((M, K, ip, ix, v, torch.from_numpy(workloads.csr_to_dense(M, K, ip, ix, v)).cuda(),
+                     torch.from_numpy(X).cuda(), torch.empty((12, M, N), device="cuda"), O.orc_csr_spmm(M, K, ip, ix, v, X)))
+    torch.cuda.synchronize()
+    failed, start, handles = [], threading.Barrier(2), []
+
+    def builds(i):
+        M, K, ip, ix, v, D, dX, dY, _ = work[i]
+        try:
+            start.wait()
+            for j in range(dY.shape[0]):
+                W = ctx.csr_from_dense_dev(D.data_ptr(), M, K) if j % 2 else ctx.csr_upload(M, K, ip, ix, v)
+                handles.append(W)
+                W.spmm_dev(dX.data_ptr(), N, dY[j].data_ptr(), mode="strict")
+        except Exception as e:
+            failed.append(repr(e))
+
+    say("two threads build on one context")
+    threads = [threading.Thread(target=builds, args=(i,)) for i in range(2)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    ctx.synchronize()
+    assert not failed, failed
+    for *_, dY, R in work:
+        for Y in dY.cpu().numpy():
+            assert np.array_equal(bits(Y), bits(R))
+    for W in handles:
+        W.free()
