@@ -1170,7 +1170,15 @@ __global__ __launch_bounds__(64 * W) void k_sp24_small(int nsteps, int nkt, cons
     struct Frag {
         v8i b[NB];
     };
+    // rows pass between the lanes of the wave here: LDS operations of a wave
+    // run in order, the fences keep the compiler to it (no instruction)
+    auto handover = [&]() {
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    };
     auto arrange = [&](Frag& g, const Slot& f, int s) {
+        handover();  // the reads of the step before come first
 #pragma unroll
         for (int h = 0; h < 2 * NB; ++h) {
             v4i b = f.b[h];
@@ -1184,6 +1192,7 @@ __global__ __launch_bounds__(64 * W) void k_sp24_small(int nsteps, int nkt, cons
                 *reinterpret_cast<v4i*>(rows + h * 1024 + wr + 16 * (wp ^ ((4 * h + (l >> 4)) & 7))) = b;
             }
         }
+        handover();
 #pragma unroll
         for (int j = 0; j < NB; ++j) {
             if constexpr (XROW) {
