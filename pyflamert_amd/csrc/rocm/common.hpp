@@ -108,6 +108,14 @@ __device__ __forceinline__ float bias_add(float v, int64_t f, const float* __res
     return bias_add_at(v, bias != nullptr ? bias + f % c_size : nullptr, beta, act);
 }
 
+// Whether two byte ranges share nothing.  A product may be given an output that
+// overlaps its activation where the activation is copied (transposed, padded)
+// before the product runs; the routes that read it in place ask this first.
+inline bool disjoint(const void* a, int64_t a_bytes, const void* b, int64_t b_bytes) {
+    const auto x = reinterpret_cast<uintptr_t>(a), y = reinterpret_cast<uintptr_t>(b);
+    return x + (uintptr_t)a_bytes <= y || y + (uintptr_t)b_bytes <= x;
+}
+
 // Grow-only device buffer owned by a context.
 struct DevBuf {
     void* p = nullptr;

@@ -1832,7 +1832,9 @@ void gemm_i8_dev(pfr_ctx* ctx, const pfr_sp24* W, const int8_t* X, int64_t N, in
     // the small tiles read X in place when its 16-byte pieces are whole, or
     // its transpose; a call that the large tiles serve in place uses no
     // scratch, and keeps it that way
-    const Plan24 plan = plan_small(ctx, W, N, 1, aligned && N % 16 == 0 && W->K > 0, xrow);
+    const int64_t ysize = out_kind == PFR_SP24_OUT_I8 ? 1 : 4;
+    const bool apart = pfr::disjoint(X, (W->K - 1) * ldx + N, Y, ysize * ((W->M - 1) * ldy + N));
+    const Plan24 plan = plan_small(ctx, W, N, 1, aligned && apart && N % 16 == 0 && W->K > 0, xrow);
     if (plan.tile >= 0) {
         const Sp24Epi ep{W->w_scale, x_scale, inv_out, out_zp, inrange, x_zp, x_u8 ? 128 : 0, xs_dev, zp_dev,
                          W->row_sum, out_kind, 0};
@@ -1966,7 +1968,8 @@ void gemm_qt_dev(pfr_ctx* ctx, const pfr_sp24* W, const uint8_t* X, bool x_u8, i
     if (small_ns < large_ns(ctx, W, T, Kp / 128, false) + 2 * kTransposeNs) {
         // the rows of X are the K-contiguous operand as they are, when their
         // 16-byte pieces are whole and aligned
-        const bool direct = W->K >= 16 && W->K % 16 == 0 && ldx % 16 == 0 && (reinterpret_cast<uintptr_t>(X) & 15) == 0;
+        const bool direct = W->K >= 16 && W->K % 16 == 0 && ldx % 16 == 0 && (reinterpret_cast<uintptr_t>(X) & 15) == 0 &&
+                            pfr::disjoint(X, (T - 1) * ldx + W->K, Y, 4 * ((T - 1) * ldy + W->M));
         const uint8_t* b = X;
         if (!direct) {
             uint8_t* xt = static_cast<uint8_t*>(ctx->scratch[3].ensure((size_t)(Np * Kp)));
@@ -2013,7 +2016,8 @@ void gemm_bf16_dev(pfr_ctx* ctx, const pfr_sp24* W, const uint16_t* X, int64_t N
     // it is transposed into a zero-padded XT (Np x Kp) first.
     const bool xrow = W->K == W->Kp && N % kI8TileN == 0 && ldx % 8 == 0 &&
                       (reinterpret_cast<uintptr_t>(X) & 15) == 0;
-    const Plan24 plan = plan_small(ctx, W, N, 2, ldx % 8 == 0 && N % 8 == 0 && W->K > 0 &&
+    const bool apart = pfr::disjoint(X, 2 * ((W->K - 1) * ldx + N), Y, 4 * ((W->M - 1) * ldy + N));
+    const Plan24 plan = plan_small(ctx, W, N, 2, ldx % 8 == 0 && N % 8 == 0 && W->K > 0 && apart &&
                                                      (reinterpret_cast<uintptr_t>(X) & 15) == 0, xrow);
     const int vec = (ldx % 4 == 0 && (reinterpret_cast<uintptr_t>(X) & 7) == 0) ? 1 : 0;
     if (plan.tile >= 0) {

@@ -2500,11 +2500,12 @@ void gemm_dev(pfr_ctx* ctx, const float* A, int64_t Mb, int64_t K, int transA, c
                          " elements, more than its workspace of " + std::to_string(ws_floats) + " floats");
         return ws;
     };
+    const bool in_place = pfr::disjoint(A, 4 * K * Mb, Y, 4 * Mb * Nf);
     if (K == 0) {
         // No terms: every output is +0 (+ bias); At is never read.
-    } else if (Mb == 1 && alpha == 1.0f) {
+    } else if (Mb == 1 && alpha == 1.0f && (transA || in_place)) {
         // one row: A is its own transpose
-    } else if (!transA && ws == nullptr && sell_serves(BT, Mb, mode == PFR_MODE_FAST) && K % 4 == 0 && aligned16(A) &&
+    } else if (!transA && ws == nullptr && in_place && sell_serves(BT, Mb, mode == PFR_MODE_FAST) && K % 4 == 0 && aligned16(A) &&
                sell_one_round(ctx, BT, Mb)) {
         // the column-slice kernel stages A's rows itself, transposed and
         // scaled on the way into LDS (the allocation-free entry keeps its
