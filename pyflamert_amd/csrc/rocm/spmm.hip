@@ -2493,18 +2493,22 @@ void gemm_dev(pfr_ctx* ctx, const float* A, int64_t Mb, int64_t K, int transA, c
     const bool pad = ws == nullptr && !transA && Mb >= kSellMinN;
     if (pad) ldt = (Mb + 3) / 4 * 4;
     hipStream_t s = ctx->stream;
-    auto tbuf = [&]() -> float* {
-        if (ws == nullptr) return static_cast<float*>(ctx->scratch[3].ensure(sizeof(float) * (size_t)(K * ldt)));
-        pfr::require(K * Mb <= ws_floats,
+    auto check_ws = [&]() {
+        pfr::require(ws == nullptr || K * Mb <= ws_floats,
                      "allocation-free Gemm: op(A) has K * Mb = " + std::to_string(K * Mb) +
                          " elements, more than its workspace of " + std::to_string(ws_floats) + " floats");
-        return ws;
+    };
+    auto tbuf = [&]() -> float* {
+        check_ws();
+        return ws ? ws : static_cast<float*>(ctx->scratch[3].ensure(sizeof(float) * (size_t)(K * ldt)));
     };
     const bool in_place = pfr::disjoint(A, 4 * K * Mb, Y, 4 * Mb * Nf);
     if (K == 0) {
         // No terms: every output is +0 (+ bias); At is never read.
     } else if (Mb == 1 && alpha == 1.0f && (transA || in_place)) {
-        // one row: A is its own transpose
+        // one row: A is its own transpose (the allocation-free entry's limit
+        // stands wherever transA == 0)
+        if (!transA) check_ws();
     } else if (!transA && ws == nullptr && in_place && sell_serves(BT, Mb, mode == PFR_MODE_FAST) && K % 4 == 0 && aligned16(A) &&
                sell_one_round(ctx, BT, Mb)) {
         // the column-slice kernel stages A's rows itself, transposed and

@@ -129,3 +129,27 @@ def test_noalloc_gemm_rejects_oversize():
     ctx.synchronize()
     BT.free()
     ctx.close()
+
+
+def test_noalloc_gemm_one_row_keeps_the_limit():
+    """One row is read as its own transpose, without the workspace; the size
+    limit holds all the same: K at the limit runs, one more is refused."""
+    import torch
+
+    from pyflamert_amd import rocm
+
+    ctx = rocm.Context(0)
+    for K in (WORKSPACE_FLOATS, WORKSPACE_FLOATS + 1):
+        BT = ctx.csr_upload(2, K, np.array([0, 2, 3]), np.array([0, K - 1, 5]), np.array([1, 2, 3], np.float32))
+        dA = torch.arange(K, dtype=torch.float32, device="cuda").remainder_(1024)
+        dY = torch.zeros(2, device="cuda")
+        torch.cuda.synchronize()
+        say(f"no-alloc Gemm of one row, K={K}")
+        if K > WORKSPACE_FLOATS:
+            with pytest.raises(_lib.InvalidArgument, match="workspace"):
+                ctx.gemm_csr_dev(dA.data_ptr(), 1, K, BT, dY.data_ptr(), noalloc=True)
+        ctx.gemm_csr_dev(dA.data_ptr(), 1, K, BT, dY.data_ptr(), noalloc=K <= WORKSPACE_FLOATS)
+        ctx.synchronize()
+        assert dY.tolist() == [2.0 * ((K - 1) % 1024), 15.0]
+        BT.free()
+    ctx.close()
