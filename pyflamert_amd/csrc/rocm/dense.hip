@@ -331,8 +331,11 @@ void gemm_dense_dev(pfr_ctx* ctx, const float* A, int64_t M, int64_t K, int tran
         const int64_t wgs = (M + tm - 1) / tm * ((N + tn - 1) / tn);
         return start + each * ((wgs + ctx->num_cu - 1) / ctx->num_cu);
     };
-    const int64_t c4 = M < (int64_t(1) << 20) ? cost(32, 32, 100, 83) : INT64_MAX;  // (grid rows)
-    const int64_t c8 = cost(64, 32, 160, 142), c16 = cost(64, 64, 240, 230), c32 = cost(128, 64, 420, 380);
+    // (A launch has fewer than 2^16 grid rows here and takes fewer than 2^32
+    // threads along x: 2^24 workgroups, N up to 2^29 in 32 columns each.)
+    const bool n32 = (N + 31) / 32 < (int64_t(1) << 24);
+    const int64_t c4 = n32 && M < (int64_t(1) << 20) ? cost(32, 32, 100, 83) : INT64_MAX;
+    const int64_t c8 = n32 ? cost(64, 32, 160, 142) : INT64_MAX, c16 = cost(64, 64, 240, 230), c32 = cost(128, 64, 420, 380);
     const int64_t best = std::min(std::min(c4, c8), std::min(c16, c32));
     if (best == c32) launch_dense<32>(ctx, a, transA != 0);
     else if (best == c16) launch_dense<16>(ctx, a, transA != 0);

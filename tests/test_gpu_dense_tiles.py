@@ -55,3 +55,19 @@ def test_dense_tiles_bit_exact(ctx, M, K, N):
             nan = np.isnan(R)
             assert np.array_equal(np.isnan(Y[:, :N]), nan)
             assert np.array_equal(Y[:, :N].view(np.uint32)[~nan], R.view(np.uint32)[~nan]), (ta, alpha)
+
+
+def test_more_columns_than_32_wide_tiles_reach(ctx):
+    """A launch takes fewer than 2^32 threads along a row of outputs: from 2^29
+    columns on only the 64-column tiles serve, also a single row."""
+    import torch
+
+    N = (1 << 29) + 5
+    B = torch.arange(N, dtype=torch.int32, device="cuda").remainder_(1 << 20).to(torch.float32)
+    Y = torch.full((N,), 7.0, device="cuda")
+    A = torch.tensor([0.75], device="cuda")
+    torch.cuda.synchronize()
+    print(f"dense 1 x 1 x {N}", flush=True)
+    ctx.gemm_dense_dev(A.data_ptr(), 1, 1, B.data_ptr(), N, Y.data_ptr())
+    ctx.synchronize()
+    assert torch.equal(Y, 0.75 * B)  # exact: 20-bit integers
