@@ -89,7 +89,10 @@ struct Outer<4> : Outer4x4 {
 // never -0 in round-to-nearest, and inf or NaN plus +0 is itself.  Tile rows
 // and columns past M and N repeat the last one and are not written.
 // AVEC: op(A) = A with 16-byte aligned rows.
-template <int NV, bool TA, bool AVEC>
+// PART: K has a chunk of its own that is not whole, or no more than two chunks: the
+// last chunk's padding is stepped over and no chunk loaded that no one reads.
+// (A product of whole chunks that carries those two branches takes 2 % longer.)
+template <int NV, bool TA, bool AVEC, bool PART>
 __global__ __launch_bounds__(256, Outer<NV>::OCC) void k_gemm_dense(
     const float* __restrict__ A, int64_t lda, const float* __restrict__ B, int64_t ldb, int64_t M, int64_t N,
     int64_t K, float alpha, const float* __restrict__ C, int64_t c_size, float beta, int act,
@@ -202,40 +205,60 @@ __global__ __launch_bounds__(256, Outer<NV>::OCC) void k_gemm_dense(
     struct Op {
         v4f a[NA], b;  // four k
     };
-    auto multiply = [&](int h) {
-        // the products of k + 1 are under way while k's are added
-        auto fetch = [&](Op& o, int k) {
+    auto fetch = [&](Op& o, int h, int k) {
 #pragma unroll
-            for (int i = 0; i < NA; ++i) o.a[i] = *reinterpret_cast<const v4f*>(&As[h][ao + i * O::AR * P + k]);
-            o.b = *reinterpret_cast<const v4f*>(&Bs[h][bo + k]);
-        };
+        for (int i = 0; i < NA; ++i) o.a[i] = *reinterpret_cast<const v4f*>(&As[h][ao + i * O::AR * P + k]);
+        o.b = *reinterpret_cast<const v4f*>(&Bs[h][bo + k]);
+    };
+    // four k: the products of k + 1 are under way while k's are added
+    auto group = [&](const Op& cur, const Op& nxt, V (&p)[NA], bool more) {
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            V n[NA];
+#pragma unroll
+            for (int i = 0; i < NA; ++i) {
+                n[i] = p[i];
+                if (u < 3) n[i] = O::mul(cur.a[i][u + 1], cur.b[u + 1]);
+                else if (more) n[i] = O::mul(nxt.a[i][0], nxt.b[0]);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int i = 0; i < NA; ++i) {
+                acc[i] = acc[i] + p[i];
+                asm volatile("" : "+v"(acc[i]));  // here, not after all the products
+                p[i] = n[i];
+            }
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    };
+    auto multiply = [&](int h) {
         Op cur;
-        fetch(cur, 0);
+        fetch(cur, h, 0);
         V p[NA];
 #pragma unroll
         for (int i = 0; i < NA; ++i) p[i] = O::mul(cur.a[i][0], cur.b[0]);
 #pragma unroll
         for (int k = 0; k < KT; k += 4) {
             Op nxt = cur;
-            if (k + 4 < KT) fetch(nxt, k + 4);
+            if (k + 4 < KT) fetch(nxt, h, k + 4);
+            group(cur, nxt, p, k + 4 < KT);
+            cur = nxt;
+        }
+    };
+    // the k positions k0 .. k1 - 1 of a chunk that is not all its own, both
+    // multiples of 4 (walking the padding too, 4096 x 4096 outputs took 62 us
+    // at K = 33 and 40 at K = 1 in 64 x 64 tiles; now 44 and 28)
+    auto multiply_part = [&](int h, int k0, int k1) {
+        Op cur;
+        fetch(cur, h, k0);
+        V p[NA];
 #pragma unroll
-            for (int u = 0; u < 4; ++u) {
-                V n[NA];
-#pragma unroll
-                for (int i = 0; i < NA; ++i) {
-                    n[i] = p[i];
-                    if (u < 3) n[i] = O::mul(cur.a[i][u + 1], cur.b[u + 1]);
-                    else if (k + 4 < KT) n[i] = O::mul(nxt.a[i][0], nxt.b[0]);
-                }
-                __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-                for (int i = 0; i < NA; ++i) {
-                    acc[i] = acc[i] + p[i];
-                    asm volatile("" : "+v"(acc[i]));  // here, not after all the products
-                    p[i] = n[i];
-                }
-                __builtin_amdgcn_sched_barrier(0);
-            }
+        for (int i = 0; i < NA; ++i) p[i] = O::mul(cur.a[i][0], cur.b[0]);
+#pragma unroll 1
+        for (int k = k0; k < k1; k += 4) {
+            Op nxt;
+            fetch(nxt, h, min(k + 4, KT - 4));  // (the last one's product is not used)
+            group(cur, nxt, p, true);
             cur = nxt;
         }
     };
@@ -243,9 +266,15 @@ __global__ __launch_bounds__(256, Outer<NV>::OCC) void k_gemm_dense(
     // 2, then chunk c + 1 goes from `nxt` into the other buffer, which was
     // last read before the previous barrier
     auto step = [&](Set& cur, const Set& nxt, int c) {
-        load(cur, c + 2);
+        if (!PART || c + 2 < nk) load(cur, c + 2);
         __builtin_amdgcn_sched_barrier(0);
-        multiply(c & 1);
+        if constexpr (PART) {
+            const int lo = c + 1 == nk ? tail : 0, hi = tiny ? (int)K : KT;
+            if (lo < 4 && hi > KT - 4) multiply(c & 1);
+            else multiply_part(c & 1, lo & ~3, (hi + 3) & ~3);
+        } else {
+            multiply(c & 1);
+        }
         if (c + 1 < nk) store(nxt, c + 1, (c + 1) & 1);
         __syncthreads();
     };
@@ -253,7 +282,7 @@ __global__ __launch_bounds__(256, Outer<NV>::OCC) void k_gemm_dense(
         Set s0, s1;
         if (tiny) load_tiny(s0);
         else load(s0, 0);
-        load(s1, 1);
+        if (!PART || nk > 1) load(s1, 1);
         store(s0, 0, 0);
         __syncthreads();
         for (int c = 0; c < nk; c += 2) {
@@ -292,12 +321,16 @@ void launch_dense(pfr_ctx* ctx, const DenseArgs& a, bool transA) {
     constexpr int TM = 2 * Outer<NV>::WM, TN = 2 * Outer<NV>::WN;
     const dim3 grid((unsigned)((a.N + TN - 1) / TN), (unsigned)((a.M + TM - 1) / TM));
     const bool avec = !transA && a.lda % 4 == 0 && a.K >= 4 && (reinterpret_cast<uintptr_t>(a.A) & 15) == 0;
-#define PFR_DENSE(T, V)                                                                                            \
-    hipLaunchKernelGGL((k_gemm_dense<NV, T, V>), grid, dim3(256), 0, ctx->stream, a.A, a.lda, a.B, a.ldb, a.M, a.N, \
+#define PFR_DENSE(T, V, P)                                                                                            \
+    hipLaunchKernelGGL((k_gemm_dense<NV, T, V, P>), grid, dim3(256), 0, ctx->stream, a.A, a.lda, a.B, a.ldb, a.M, a.N, \
                        a.K, a.alpha, a.C, a.c_size, a.beta, a.act, a.Y, a.ldy)
-    if (transA) PFR_DENSE(true, false);
-    else if (avec) PFR_DENSE(false, true);
-    else PFR_DENSE(false, false);
+    const bool part = a.K % Outer<NV>::KT != 0 || a.K <= 2 * Outer<NV>::KT;
+    if (transA && part) PFR_DENSE(true, false, true);
+    else if (transA) PFR_DENSE(true, false, false);
+    else if (avec && part) PFR_DENSE(false, true, true);
+    else if (avec) PFR_DENSE(false, true, false);
+    else if (part) PFR_DENSE(false, false, true);
+    else PFR_DENSE(false, false, false);
 #undef PFR_DENSE
 }
 
@@ -316,26 +349,30 @@ void gemm_dense_dev(pfr_ctx* ctx, const float* A, int64_t M, int64_t K, int tran
         c_size = 0;
     }
     const DenseArgs a{A, transA ? M : K, B, ldb, M, N, K, alpha, C, c_size, beta, act, Y, ldy};
-    // The tile with the least estimated time: workgroups per CU times the
-    // tile's cost, plus its start.  Small tiles give a small product more
-    // waves (a sum is a chain over all of K, so K cannot be split) and let
+    // The tile with the least estimated time.  Small tiles give a small product
+    // more waves (a sum is a chain over all of K, so K cannot be split) and let
     // the MFMAs of one wave run beside the adds of another: within one wave
     // they take turns (205 clocks per k at NV = 32 against 134 with two waves
-    // per SIMD).  Large ones read their operands less often.  Measured with K
-    // = 768 (us; NV = 4 / 8 / 16 / 32): 64 x 768 outputs 19.0 / 29.8 / 47.6 /
-    // 83.7, 512 x 3072 63.5 / 59.0 / 64.1 / 88.6, 1024 x 3072 113.9 / 104.2 /
-    // 103.8 / 117.0, and 2048 cubed 357 / 320 / 292 / 277.  (Before, with the
-    // multiplies and adds both on the vector unit and one 64 x 64 tile: 117,
-    // 125, 169 and 448.)
-    auto cost = [&](int64_t tm, int64_t tn, int64_t start, int64_t each) {
-        const int64_t wgs = (M + tm - 1) / tm * ((N + tn - 1) / tn);
-        return start + each * ((wgs + ctx->num_cu - 1) / ctx->num_cu);
+    // per SIMD).  Large ones read their operands less often.  A k takes k1[n - 1]
+    // ns on a CU that holds n workgroups, up to four, and four at a time where
+    // there are more (an odd one on NV = 32 runs half alone); a workgroup
+    // takes `each` ns besides, for its start and its outputs.  Measured over 64 x
+    // 768 to 4096 x 4096 outputs and K from 1 to 2048; with K = 768 (us; NV = 4 /
+    // 8 / 16 / 32): 64 x 768 outputs 19.4 / 31.0 / 48.0 / 83.8, 512 x 3072 56.1 /
+    // 55.0 / 59.2 / 84.7, 1000 x 4096 138 / 122 / 115 / 110, 2048 x 3072 204 / 181 /
+    // 168 / 188, and 2048 cubed 357 / 320 / 292 / 277; with K = 16: 4096 x 4096 53 /
+    // 38 / 33 / 39.  (With the multiplies and adds both on the vector unit and one
+    // 64 x 64 tile: 117, 118, 162, 234, 448 and 31.)
+    auto cost = [&](int64_t tm, int64_t tn, int64_t each, const int (&k1)[4]) {
+        const int64_t wgs = (M + tm - 1) / tm * ((N + tn - 1) / tn), n = (wgs + ctx->num_cu - 1) / ctx->num_cu;
+        return n * each + K * (n / 4 * k1[3] + (n % 4 ? k1[n % 4 - 1] : 0));
     };
     // (A launch has fewer than 2^16 grid rows here and takes fewer than 2^32
     // threads along x: 2^24 workgroups, N up to 2^29 in 32 columns each.)
     const bool n32 = (N + 31) / 32 < (int64_t(1) << 24);
-    const int64_t c4 = n32 && M < (int64_t(1) << 20) ? cost(32, 32, 100, 83) : INT64_MAX;
-    const int64_t c8 = n32 ? cost(64, 32, 160, 142) : INT64_MAX, c16 = cost(64, 64, 240, 230), c32 = cost(128, 64, 420, 380);
+    const int64_t c4 = n32 && M < (int64_t(1) << 20) ? cost(32, 32, 600, {19, 23, 35, 42}) : INT64_MAX;
+    const int64_t c8 = n32 ? cost(64, 32, 750, {34, 40, 63, 75}) : INT64_MAX;
+    const int64_t c16 = cost(64, 64, 1450, {55, 68, 110, 136}), c32 = cost(128, 64, 3500, {100, 129, 226, 257});
     const int64_t best = std::min(std::min(c4, c8), std::min(c16, c32));
     if (best == c32) launch_dense<32>(ctx, a, transA != 0);
     else if (best == c16) launch_dense<16>(ctx, a, transA != 0);
