@@ -1699,7 +1699,13 @@ void check_i8(const pfr_sp24* W) {
 // per CU * (each + steps * step).  Fitted to 4096 x {4096, 11008} on 1 .. 512
 // columns with 8 rotating weights (int8, x . W form); for instance 4096 x 4096
 // on 64 columns: 9.9 us in 16 x 16 tiles, 7.7 in 32 x 16, 7.0 in 32 x 32, 8.5
-// in 64 x 32 and 11.8 in 64 x 64; on 512: 57, 43, 43, 28 and 17.
+// in 64 x 32 and 11.8 in 64 x 64; on 512: 57, 43, 43, 28 and 17.  The three
+// corrections below, and those of the large tiles, were set so that over 576
+// products (int8, uint8, bf16 and x . W; M 768 .. 22016, K 768 .. 11008, 8 .. 2000
+// columns; every route of each timed) none takes a route that is more than 3 %
+// slower than the large tiles, and few give up more than a microsecond against
+// the best one.  (Without them 27 of the 576 did, on 200 and more columns: 4096 x
+// 11008 int8 on 1024 columns 89 us against 49, bf16 on 1000 141 against 86.)
 struct SmallTile {
     int rb, nb, w, start, each, step;
 };
@@ -1709,21 +1715,26 @@ constexpr SmallTile kSmallTiles[] = {{1, 1, 8, 3500, 870, 24},
                                      {4, 2, 8, 2500, 3400, 96},
                                      {4, 4, 4, 6000, 2000, 140}};
 
-// The tile (an index into kSmallTiles) that serves an M x N product of
-// `steps` 128-byte steps soonest, and its time in ns.  elem: 0 for XT, else
-// the element size of a row-major X read in place: then a tile narrower than
-// the rows reads pieces of lines (4096 x 4096 int8 on 128 columns: 64 x 32
-// tiles 13.0 us, against 7.3 after a transpose of 4), so only tiles as wide as
-// the rows, or the widest, are taken.
-int small_tile(const pfr_ctx* ctx, int64_t M, int64_t N, int64_t steps, int elem, int64_t* ns) {
+// The tile (an index into kSmallTiles) that serves a product on N columns in
+// `steps` 128-byte steps soonest, and its time in ns.  in_place: X is read
+// row-major; then a tile narrower than the rows reads pieces of lines (4096 x
+// 4096 int8 on 128 columns: 64 x 32 tiles 13.0 us, against 7.3 after a transpose
+// of 4), so only tiles as wide as the rows, or the widest, are taken, and the
+// widest's steps take 170 ns.  Every workgroup reads its columns of X anew, so
+// steps slow down as X outgrows an XCD's 4 MiB L2.
+int small_tile(const pfr_ctx* ctx, const pfr_sp24* W, int64_t N, int64_t steps, bool in_place, int64_t* ns) {
+    const bool bf = W->dtype == PFR_BF16;
+    const double spill = (double)W->K * (double)N * (bf ? 2 : 1) / (4 << 20) - 1;
+    const double slow = 1 + (bf ? 0.1 : 0.25) * std::max(0.0, spill);
     int best = 0;
     *ns = INT64_MAX;
     for (int i = 0; i < 5; ++i) {
         const SmallTile& t = kSmallTiles[i];
-        if (elem > 0 && t.nb < 4 && 16 * t.nb < N) continue;
-        const int64_t wgs = (M + 16 * t.rb - 1) / (16 * t.rb) * ((N + 16 * t.nb - 1) / (16 * t.nb));
+        if (in_place && t.nb < 4 && 16 * t.nb < N) continue;
+        const int64_t wgs = (W->M + 16 * t.rb - 1) / (16 * t.rb) * ((N + 16 * t.nb - 1) / (16 * t.nb));
         const int64_t per_cu = (wgs + ctx->num_cu - 1) / ctx->num_cu;
-        const int64_t e = t.start + per_cu * (t.each + steps * t.step);
+        const double step = in_place && t.nb == 4 ? 170 : t.step;
+        const int64_t e = t.start + per_cu * (t.each + (int64_t)((double)steps * step * slow));
         if (e < *ns) *ns = e, best = i;
     }
     return best;
@@ -1732,15 +1743,22 @@ int small_tile(const pfr_ctx* ctx, int64_t M, int64_t N, int64_t steps, int elem
 // The large-tile kernels' time in ns: a start and so much per 128-byte step
 // and round, more when more tiles share the memory (measured: int8 from
 // row-major X 18.7 us at 16 and 22.8 at 172 tiles, K = 4096; from XT 22 and
-// 29; bf16 29 and 38).  And that of transposing the activation first.
-int64_t large_ns(const pfr_ctx* ctx, const pfr_sp24* W, int64_t N, int64_t steps, bool xrow) {
+// 29; bf16 29 and 38), less from XT where the rows of X and Y are whole 16-byte
+// pieces (`whole`; int8, K = 4096: 24 us at 129 tiles, against 30 at 86 without).
+// A last round that is nearly empty costs less than a full one.  uint8 values
+// pass through a sign flip first.
+int64_t large_ns(const pfr_ctx* ctx, const pfr_sp24* W, int64_t N, int64_t steps, bool xrow, bool u8, bool whole) {
     const int64_t tiles = W->Mp / kI8TileM * ((N + kI8TileN - 1) / kI8TileN);
-    const int64_t rounds = (tiles + ctx->num_cu - 1) / ctx->num_cu, busy = std::min<int64_t>(tiles, ctx->num_cu);
+    const int64_t full = (tiles + ctx->num_cu - 1) / ctx->num_cu, busy = std::min<int64_t>(tiles, ctx->num_cu);
+    const double rounds = full > 1 ? 0.75 * (double)full + 0.25 * (double)tiles / ctx->num_cu : 1;
     const int64_t step = W->dtype == PFR_BF16 ? std::min<int64_t>(380 + 9 * busy / 2, 600)
                                               : (xrow ? 430 + 7 * busy / 10 : 500 + 14 * busy / 10);
-    return 5000 + rounds * steps * step;
+    const double scale = W->dtype == PFR_I8 && !xrow && whole ? 0.85 : 1;
+    const int64_t start = W->dtype == PFR_BF16 ? 6000 : 5000;
+    return start + (u8 ? 3000 : 0) + (int64_t)(rounds * (double)(steps * step) * scale);
 }
-constexpr int64_t kTransposeNs = 4000;
+// That of transposing, padding or flipping `bytes` into a copy first.
+int64_t transpose_ns(int64_t bytes) { return 4000 + bytes / 5000; }
 
 // How a W . X product runs: on the small tile `tile` (-1: the large ones),
 // reading X in place or its transpose.  pieces: X can be read in place by the
@@ -1750,16 +1768,17 @@ struct Plan24 {
     int tile;
     bool in_place;
 };
-Plan24 plan_small(const pfr_ctx* ctx, const pfr_sp24* W, int64_t N, int elem, bool pieces, bool xrow) {
-    const int64_t kstep = 128 / elem, steps = (W->K + kstep - 1) / kstep;
-    int64_t best = large_ns(ctx, W, N, W->Kp / kstep, xrow) + (xrow ? 0 : kTransposeNs), ns = 0;
+Plan24 plan_small(const pfr_ctx* ctx, const pfr_sp24* W, int64_t N, int elem, bool pieces, bool xrow, bool u8,
+                  bool whole) {
+    const int64_t kstep = 128 / elem, steps = (W->K + kstep - 1) / kstep, transpose = transpose_ns(W->K * N * elem);
+    int64_t best = large_ns(ctx, W, N, W->Kp / kstep, xrow, u8, whole) + (xrow ? 0 : transpose), ns = 0;
     Plan24 p{-1, false};
     if (!xrow) {
-        const int t = small_tile(ctx, W->M, N, steps, 0, &ns);
-        if (ns + kTransposeNs < best) best = ns + kTransposeNs, p = {t, false};
+        const int t = small_tile(ctx, W, N, steps, false, &ns);
+        if (ns + transpose < best) best = ns + transpose, p = {t, false};
     }
     if (pieces) {
-        const int t = small_tile(ctx, W->M, N, steps, elem, &ns);
+        const int t = small_tile(ctx, W, N, steps, true, &ns);
         if (ns < best) p = {t, true};
     }
     return p;
@@ -1834,7 +1853,8 @@ void gemm_i8_dev(pfr_ctx* ctx, const pfr_sp24* W, const int8_t* X, int64_t N, in
     // scratch, and keeps it that way
     const int64_t ysize = out_kind == PFR_SP24_OUT_I8 ? 1 : 4;
     const bool apart = pfr::disjoint(X, (W->K - 1) * ldx + N, Y, ysize * ((W->M - 1) * ldy + N));
-    const Plan24 plan = plan_small(ctx, W, N, 1, aligned && apart && N % 16 == 0 && W->K > 0, xrow);
+    const Plan24 plan = plan_small(ctx, W, N, 1, aligned && apart && N % 16 == 0 && W->K > 0, xrow, x_u8,
+                                   aligned && N % 16 == 0 && ldy % 16 == 0);
     if (plan.tile >= 0) {
         const Sp24Epi ep{W->w_scale, x_scale, inv_out, out_zp, inrange, x_zp, x_u8 ? 128 : 0, xs_dev, zp_dev,
                          W->row_sum, out_kind, 0};
@@ -1964,8 +1984,10 @@ void gemm_qt_dev(pfr_ctx* ctx, const pfr_sp24* W, const uint8_t* X, bool x_u8, i
     if (!xs_dev) pfr::require(x_scale > 0.0f && std::isfinite(x_scale), "x_scale must be positive and finite");
     const int64_t Kp = W->Kp, Np = round_up(T, kI8TileN), ldyp = round_up(T, 16);
     int64_t small_ns = 0;
-    const int tile = small_tile(ctx, W->M, T, (W->K + 127) / 128, 0, &small_ns);
-    if (small_ns < large_ns(ctx, W, T, Kp / 128, false) + 2 * kTransposeNs) {
+    const int tile = small_tile(ctx, W, T, (W->K + 127) / 128, false, &small_ns);
+    // (the large tiles read X padded and leave the product to be transposed)
+    const int64_t copies = transpose_ns(T * W->K) + transpose_ns(4 * W->M * T);
+    if (small_ns < large_ns(ctx, W, T, Kp / 128, false, false, false) + copies) {
         // the rows of X are the K-contiguous operand as they are, when their
         // 16-byte pieces are whole and aligned
         const bool direct = W->K >= 16 && W->K % 16 == 0 && ldx % 16 == 0 && (reinterpret_cast<uintptr_t>(X) & 15) == 0 &&
@@ -2018,7 +2040,7 @@ void gemm_bf16_dev(pfr_ctx* ctx, const pfr_sp24* W, const uint16_t* X, int64_t N
                       (reinterpret_cast<uintptr_t>(X) & 15) == 0;
     const bool apart = pfr::disjoint(X, 2 * ((W->K - 1) * ldx + N), Y, 4 * ((W->M - 1) * ldy + N));
     const Plan24 plan = plan_small(ctx, W, N, 2, ldx % 8 == 0 && N % 8 == 0 && W->K > 0 && apart &&
-                                                     (reinterpret_cast<uintptr_t>(X) & 15) == 0, xrow);
+                                                     (reinterpret_cast<uintptr_t>(X) & 15) == 0, xrow, false, false);
     const int vec = (ldx % 4 == 0 && (reinterpret_cast<uintptr_t>(X) & 7) == 0) ? 1 : 0;
     if (plan.tile >= 0) {
         if (plan.in_place) {

@@ -1,8 +1,10 @@
-"""The small-tile 2:4 kernel (few columns or few tiles): every tile it has, the
-remainders of its rows, columns and k steps, waves without a step, and each
-form that runs on it: int8 W.X with the three outputs, uint8 with a zero point
-(host value and device scalar), the x.W form from aligned rows and through the
-padded copy, and bf16.
+"""The small-tile 2:4 kernel (few columns or few tiles): every tile it has, from
+the activation's transpose and reading it in place, the remainders of its
+rows, columns and k steps, waves without a step, and each form that runs on
+it: int8 W.X with the three outputs, uint8 with a zero point (host value and
+device scalar), the x.W form from aligned rows and through the padded copy,
+and bf16, with non-finite values in the last k row too.
+test_dispatch_coverage.py checks that the shapes reach every tile in each form.
 
 Bar: int32 and requantised int8 exact, float outputs exact to the bit (the
 exact accumulator times RN(w_scale * x_scale), quant_ops.cpp:435); bf16 within
@@ -17,7 +19,8 @@ pytestmark = pytest.mark.gpu
 # tiles of 16 x 16, 32 x 16, 32 x 32, 64 x 32 and 64 x 64 outputs; K of one
 # step or less, of fewer steps than waves, and of no whole step
 SHAPES = [(1, 4, 1), (17, 100, 3), (100, 500, 17), (300, 1156, 16), (4100, 608, 9), (4096, 1024, 64),
-          (3985, 900, 49), (4096, 1040, 128), (4000, 512, 121), (4096, 1028, 200), (4033, 640, 195), (1088, 640, 512)]
+          (3985, 900, 49), (4096, 1040, 128), (4000, 512, 121), (4096, 1028, 200), (4033, 640, 195), (1088, 640, 512),
+          (17000, 100, 16), (500, 272, 32), (12000, 100, 16), (3001, 640, 65)]
 
 
 @pytest.fixture(scope="module")
@@ -49,16 +52,17 @@ def test_int8(ctx, M, K, N):
         p = workloads.round_half_away(f * (np.float32(1.0) / np.float32(out_scale)))
         r = np.clip(p.astype(np.int64) + zp, -128, 127).astype(np.int8)
         assert np.array_equal(W.gemm_i8(X, x_scale=0.05, out="i8", out_scale=out_scale, out_zp=zp), r)
-    # a uint8 activation with a zero point, columns inside wider rows
-    U = rng.integers(0, 256, (K, N + 5)).astype(np.uint8)
-    accu = (q.astype(np.float64) @ (U[:, :N].astype(np.float64) - 77)).astype(np.int64)
-    dU = torch.from_numpy(U).cuda()
-    dY = torch.full((M, N + 3), -1, dtype=torch.int32, device="cuda")
-    torch.cuda.synchronize()
-    W.gemm_q_dev(dU.data_ptr(), True, N, dY.data_ptr(), x_zp=77, out="i32", ldx=N + 5, ldy=N + 3)
-    ctx.synchronize()
-    Y = dY.cpu().numpy()
-    assert np.array_equal(Y[:, :N], accu.astype(np.int32)) and (Y[:, N:] == -1).all()
+    # a uint8 activation with a zero point, columns inside wider rows and not
+    for ldx, ldy in ((N + 5, N + 3), (N, N)):
+        U = rng.integers(0, 256, (K, ldx)).astype(np.uint8)
+        accu = (q.astype(np.float64) @ (U[:, :N].astype(np.float64) - 77)).astype(np.int64)
+        dU = torch.from_numpy(U).cuda()
+        dY = torch.full((M, ldy), -1, dtype=torch.int32, device="cuda")
+        torch.cuda.synchronize()
+        W.gemm_q_dev(dU.data_ptr(), True, N, dY.data_ptr(), x_zp=77, out="i32", ldx=ldx, ldy=ldy)
+        ctx.synchronize()
+        Y = dY.cpu().numpy()
+        assert np.array_equal(Y[:, :N], accu.astype(np.int32)) and (Y[:, N:] == -1).all()
 
 
 @pytest.mark.parametrize("M,K,T", SHAPES)
@@ -103,3 +107,12 @@ def test_bf16(ctx, M, K, N):
     n = K // 2 + 8  # terms, and the sums across waves
     bound = n * 2.0 ** -24 / (1 - n * 2.0 ** -24) * (np.abs(w) @ np.abs(x))
     assert (np.abs(Y - w @ x) <= bound + 1e-30).all()
+    # inf and NaN in the last k row: the rows read past it (K is no whole step)
+    # must not repeat it against the packing's zeros
+    xi = xb.copy()
+    xi[K - 1, 0], xi[K - 1, N // 2] = 0x7F80, 0x7FC0
+    odd = np.zeros(N, bool)
+    odd[[0, N // 2]] = True
+    Z = W.gemm_bf16(xi).astype(np.float64)
+    assert np.array_equal(Z[:, ~odd], Y[:, ~odd])
+    assert np.array_equal(~np.isfinite(Z[:, odd]), np.repeat(w[:, K - 1:] != 0, odd.sum(), axis=1))
