@@ -2175,15 +2175,22 @@ void launch_sell_w(pfr_ctx* ctx, const pfr_csr* Wt, const float* X, int N, int64
 // count with the fewest estimated clocks runs, the larger on a tie.  (12 waves
 // fill the chip where 16 leave a quarter of it idle, 8 need a second round:
 // 3001 x 5003 on 256 columns 48.0 -> 41.5 us, 768 x 3072 on 1024 53.0 -> 48.2,
-// 768 x 768 on 1024 15.4 -> 13.5.)  The same rule holds for a weight of one
-// chunk, several of whose workgroups share a CU.  Fewer than four waves lose:
-// each wave then stages more of X than it walks.
-int sell_waves(const pfr_ctx* ctx, const pfr_csr* Wt, int64_t N, int64_t* rounds_out = nullptr) {
+// 768 x 768 on 1024 15.4 -> 13.5.)  Fewer than four waves lose: each wave then
+// stages more of X than it walks.
+// Two or three workgroups of a weight of one chunk share a CU.  The rule mostly
+// stays within 5 % of the best count there (512 x 784 to 11008 x 768 on 16 to 2048
+// columns, strict and fast).  It does not in many rounds of 16 waves: 11008 x 768,
+// 10 %, on 1024 columns takes 78 us strict and 80 fast in 16 waves, 68 and 59 in
+// 12.  A Gemm's outputs (`strided`: consecutive rows of W a float apart) leave
+// sooner from 8 there (strict 171 us in 16 waves, 154 in 8; the launch with two
+// buffers, one workgroup per CU, took 160), so it runs them.
+int sell_waves(const pfr_ctx* ctx, const pfr_csr* Wt, int64_t N, bool strided, int64_t* rounds_out = nullptr) {
     const int64_t slices = (N + pfr::kSellCols - 1) / pfr::kSellCols;
     auto rounds = [&](int64_t w) { return ((Wt->sell_nslab + w - 1) / w * slices + ctx->num_cu - 1) / ctx->num_cu; };
     const int64_t c16 = rounds(16) * 214, c12 = rounds(12) * 174, c8 = rounds(8) * 130, c4 = rounds(4) * 100;
     const int64_t best = std::min(std::min(c16, c12), std::min(c8, c4));
-    const int w = best == c16 ? 16 : (best == c12 ? 12 : (best == c8 ? 8 : 4));
+    int w = best == c16 ? 16 : (best == c12 ? 12 : (best == c8 ? 8 : 4));
+    if (w == 16 && strided && Wt->sell_nch == 1 && rounds(16) >= 3) w = 8;
     if (rounds_out) *rounds_out = rounds(w);
     return w;
 }
@@ -2194,7 +2201,7 @@ void launch_sell_x(pfr_ctx* ctx, const pfr_csr* Wt, const float* X, int N, int64
                    float alpha) {
 #define PFR_SELLW(WV) \
     launch_sell_w<FAST, XVEC, WV, XT, NF>(ctx, Wt, X, N, ldx, nx, Y, ldy_r, ldy_c, yvec, bias, c_size, beta, act, alpha)
-    const int w = sell_waves(ctx, Wt, N);
+    const int w = sell_waves(ctx, Wt, N, ldy_c != 1);
     if (w == 16) PFR_SELLW(16);
     else if (w == 12) PFR_SELLW(12);
     else if (w == 8) PFR_SELLW(8);
@@ -2401,7 +2408,7 @@ bool sell_serves(const pfr_csr* W, int64_t N, bool fast) {
 // chunks would fall to the staging wave alone).
 bool sell_one_round(const pfr_ctx* ctx, const pfr_csr* W, int64_t N) {
     int64_t rounds = 0;
-    const int w = sell_waves(ctx, W, N, &rounds);
+    const int w = sell_waves(ctx, W, N, true, &rounds);
     return rounds == 1 && (w >= 12 || W->sell_nch == 1);
 }
 
@@ -2516,8 +2523,10 @@ void gemm_dev(pfr_ctx* ctx, const float* A, int64_t Mb, int64_t K, int transA, c
         // workspace copy and the size limit it states).  Its workgroups
         // stage through registers, more slowly than the direct-to-LDS copy of
         // a transposed A, so this pays off when the launch runs in one round
-        // (every workgroup stages once, side by side): 768 x 768 at 1024
-        // tokens 26.0 -> 21.7 us; 3072 x 768 (three rounds) 66.1 -> 67.8 us.
+        // (every workgroup stages once, side by side): 768 x 768, 20 %, at 1024
+        // tokens 22.4 -> 17.2 us; 3072 x 768 (three rounds) 46.0 -> 53.8 us.  (A
+        // weight of one chunk gains in two rounds too, 768 x 768 at 2048 tokens
+        // 34.4 -> 31.1, and loses 6 % on 16 to 64 tokens, 10.6 -> 11.3.)
         launch_spmm(ctx, BT, A, Mb, K, Y, 1, Nf, C, c_size, beta, mode == PFR_MODE_FAST, act, false, true, alpha);
         return;
     } else if (!transA) {

@@ -25,6 +25,7 @@ def ctx():
     (700, 768, (9, 11, 12, 15, 1023)),  # one chunk
     (768, 1500, (13, 1024)),            # two chunks, 12 waves at 1024
     (3001, 2049, (9, 37, 99, 130, 255)),
+    (3070, 250, (1024,)),               # one chunk, 8 waves in the Gemm form for its many rounds
     (40, 3000, (10, 33))])
 def test_widths(ctx, M, K, widths):
     import torch
