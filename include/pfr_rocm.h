@@ -159,11 +159,15 @@ int pfr_csr_info(const pfr_csr* w, int64_t* M, int64_t* K, int64_t* nnz);
  * (fast, N <= 8) are built by the
  * first product through the handle that would use one: that call plans on
  * the host, allocates, fills on the device and synchronizes the handle's
- * stream.  While that stream is being captured into a graph, and in
+ * stream.  The sliced-ELL copy of an int8 weight, or for 9 to 15 columns, is
+ * built later: by the product at which the time lost without it, as estimated,
+ * comes to three quarters of the build's (the first or second for long rows
+ * and many columns, one after tens for short rows and few).
+ * While that stream is being captured into a graph, and in
  * pfr_gemm_csr_act_noalloc_dev, nothing is built and a product without its
  * copy runs a kernel that reads the CSR in place (same results in strict
  * mode, the fast mode's own rounding otherwise), so run each kind of
- * product once before capture.  No counterpart in the reference (its
+ * product before capture, once or until this figure has grown.  No counterpart in the reference (its
  * weights are host memory); for footprint reports. */
 int pfr_csr_device_bytes(const pfr_csr* w, int64_t* bytes);
 int pfr_csr_free(pfr_csr* w);

@@ -288,13 +288,17 @@ struct pfr_csr {
     uint64_t* pattern = nullptr;
     int64_t pattern_nw = 0;
     // The sliced-ELL, row-chain and balanced copies are built on the first
-    // product that would use them (pfr::csr_build_copies): `pending` holds
+    // product that would use them, or, for a sliced-ELL copy that another kernel
+    // can do without, on a later one (pfr::csr_build_copies): `pending` holds
     // the pfr::kCopy* bits of those still to build, and the host keeps what
     // their plans need -- the row pointers and the per-row counts of each
     // copy's column chunks (M x a few integers; empty when that copy is not
     // wanted).  Freed when nothing is pending.
     std::atomic<uint32_t> pending{0};
     std::mutex lazy_mu;
+    // What products that read the CSR in place took longer than on a sliced-ELL
+    // copy still to be built (ns, estimated; strict and fast): see ensure_copies.
+    std::atomic<int64_t> sell_owed[2] = {{0}, {0}};
     std::vector<int32_t> h_rowptr, h_sell_cnt, h_bal_cnt;
     // Device bytes the handle holds (every array above).
     int64_t dev_bytes = 0;

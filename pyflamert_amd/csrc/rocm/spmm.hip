@@ -2451,14 +2451,54 @@ void check_act(int act) {
     pfr::require(act == PFR_ACT_NONE || act == PFR_ACT_RELU || act == PFR_ACT_GELU, "unknown activation");
 }
 
+// Estimates in ns, to a factor of two: building a sliced-ELL copy, and what a
+// product of N columns loses while it reads the CSR in place.  The build: its
+// fixed steps, the plan's sorts over the rows' chunk counts, the entries'
+// allocation and fill and, in fast mode, the choice of each chunk's order, a chain
+// over its longest row (measured: 4096 x 4096, 10 %, lognormal rows 490 us strict
+// and 690 fast; 768 x 768, 20 % 57 and 320; 11008 x 4096, 5 % 860 and 1120).  In
+// place a wave or less walks a row, so the longest takes 62 ns per nonzero (75 and
+// 95 in the kernels for 64 and more columns, per 64 or 256 of them); on the copy
+// it takes 24, once per round (12 columns of the three weights: 169, 35 and 72 us
+// in place, 69, 16 and 31 on the copy).
+int64_t sell_build_ns(const pfr_csr* W, bool fast) {
+    const int64_t nch = (W->K + pfr::kSellMaxKC - 1) / pfr::kSellMaxKC;
+    const int64_t run = std::min<int64_t>(W->max_row_nnz * 4 / 3 / nch, pfr::kSellMaxKC);
+    return 20000 + W->M * (40 + 12 * nch) + W->nnz * (fast ? 10 : 6) / 100 + (fast ? 400 * run : 0);
+}
+int64_t sell_saving_ns(const pfr_ctx* ctx, const pfr_csr* W, int64_t N, bool fast, bool strided) {
+    const int64_t slices = (N + pfr::kSellCols - 1) / pfr::kSellCols, slabs = (W->M + pfr::kSellRows - 1) / pfr::kSellRows;
+    const int64_t copy = 24 * W->max_row_nnz * std::max<int64_t>(1, slices * slabs / (16 * ctx->num_cu));
+    if (sell_runs(W, fast) != nullptr) return copy / 5;  // the storage-order copy serves, more slowly than the fast one
+    const bool vec = N % 4 == 0 && !strided;
+    const int64_t passes = N < 64 ? 1 : (vec ? (N + 255) / 256 : (N + 63) / 64);
+    const int64_t row = N < 64 ? 62 : (vec ? 95 : 75);
+    return passes * std::max<int64_t>(row * W->max_row_nnz, W->nnz * 3 / 100) - copy;
+}
+
 // Builds the derived copy that a product of N columns in this mode runs on,
-// when the handle still has it pending (its first such product).
-void ensure_copies(const pfr_ctx* ctx, const pfr_csr* W, int64_t N, bool fast) {
+// when the handle still has it pending: on its first such product, but for the
+// sliced-ELL copy of products that a kernel can also serve from the CSR well
+// enough (int8 weights, whose copy is also large, and fewer than kSellAtOnceN
+// columns).  There the estimated ns that in-place products lose add up, and the
+// copy is built when they come to three quarters of its cost: a handle used a few
+// times does not pay for it (the first product of the 11008 x 4096 weight above on
+// 12 columns takes 126 us strict and 118 fast instead of 1051 and 1180), and one
+// used often has lost no more than about the build's time without it.
+constexpr int64_t kSellAtOnceN = 16;
+void ensure_copies(const pfr_ctx* ctx, const pfr_csr* W, int64_t N, bool fast, bool strided) {
+    const uint32_t pending = W->pending.load(std::memory_order_acquire);
     uint32_t need = 0;
-    if (N >= kSellMinN) need |= fast ? pfr::kCopySellFast : pfr::kCopySell;
     if (fast && ((N >= 2 && N <= 8) || (N == 1 && !(ctx->merge && W->mp_wave != nullptr)))) need |= pfr::kCopyBal;
     if (!fast && N <= 8) need |= pfr::kCopyChain;
-    if ((W->pending.load(std::memory_order_acquire) & need) != 0) pfr::csr_build_copies(const_cast<pfr_csr*>(W), need);
+    const uint32_t sell = N >= kSellMinN ? (fast ? pfr::kCopySellFast : pfr::kCopySell) & pending : 0;
+    if (sell != 0 && W->vdt == PFR_F32 && N >= kSellAtOnceN) need |= sell;
+    else if (sell != 0) {
+        auto& owed = const_cast<pfr_csr*>(W)->sell_owed[fast ? 1 : 0];
+        const int64_t saving = std::max<int64_t>(0, sell_saving_ns(ctx, W, N, fast, strided));
+        if (4 * (owed.fetch_add(saving) + saving) >= 3 * sell_build_ns(W, fast)) need |= sell;
+    }
+    if ((pending & need) != 0) pfr::csr_build_copies(const_cast<pfr_csr*>(W), need);
 }
 
 void spmm_dev(pfr_ctx* ctx, const pfr_csr* W, const float* X, int64_t N, int64_t ldx, float* Y,
@@ -2469,7 +2509,7 @@ void spmm_dev(pfr_ctx* ctx, const pfr_csr* W, const float* X, int64_t N, int64_t
     pfr::require(mode == PFR_MODE_STRICT || mode == PFR_MODE_FAST, "unknown mode");
     pfr::require((X && Y) || W->M * N == 0, "null X/Y");
     check_act(act);
-    if (W->M > 0 && N > 0) ensure_copies(ctx, W, N, mode == PFR_MODE_FAST);
+    if (W->M > 0 && N > 0) ensure_copies(ctx, W, N, mode == PFR_MODE_FAST, false);
     launch_spmm(ctx, W, X, N, ldx, Y, ldy, 1, nullptr, 0, 0.0f, mode == PFR_MODE_FAST, act);
 }
 
@@ -2487,7 +2527,7 @@ void gemm_dev(pfr_ctx* ctx, const float* A, int64_t Mb, int64_t K, int transA, c
     const int64_t Nf = BT->M;
     if (Mb == 0 || Nf == 0) return;
     pfr::require(A != nullptr && Y != nullptr, "null A/Y");
-    if (ws == nullptr) ensure_copies(ctx, BT, Mb, mode == PFR_MODE_FAST);  // the allocation-free entry builds none
+    if (ws == nullptr) ensure_copies(ctx, BT, Mb, mode == PFR_MODE_FAST, true);  // the allocation-free entry builds none
     if (C == nullptr || c_size <= 0) {
         C = nullptr;
         c_size = 0;

@@ -3,7 +3,8 @@ starts with the CSR itself (uint16 columns when K <= 65536, values, row
 pointers, row scales), the row-block table and the merge-path partition;
 the first product that runs on the nnz-balanced copy (fast, 2 <= N <= 8),
 the row-chain copy (strict, N <= 8) or the sliced-ELL copy (float32,
-N >= 16) builds it, and later products reuse it.  Products match the oracle
+N >= 16) builds it, and later products reuse it; int8 weights and 9 to 15
+columns build theirs after some products in place.  Products match the oracle
 as everywhere else (strict bit for bit, fast within 1e-5 normwise).  A
 product captured into a HIP graph while its copy is still pending builds
 nothing and reads the CSR in place: in strict mode the same bits as the
@@ -200,10 +201,17 @@ def test_allocation_free_products_beside_a_build(ctx, values, Mb):
 
         def build():
             try:
-                for mode in ("strict", "fast"):
-                    Y = W.spmm(X, mode=mode)
-                    if mode == "strict" and not np.array_equal(bits(Y), bits(R.T)):
-                        failed.append("the building product")
+                # (fast products would do with the strict copy for long)
+                for mode in ("fast", "strict"):
+                    b = W.device_bytes()
+                    for _ in range(60):
+                        Y = W.spmm(X, mode=mode)
+                        if mode == "strict" and not np.array_equal(bits(Y), bits(R.T)):
+                            failed.append("the building product")
+                        if W.device_bytes() > b:
+                            break
+                    else:
+                        failed.append(f"no copy: {mode}")
             except Exception as e:
                 failed.append(repr(e))
             finally:
@@ -269,4 +277,36 @@ def test_two_threads_build_on_one_context(ctx):
         for Y in dY.cpu().numpy():
             assert np.array_equal(bits(Y), bits(R))
     for W in handles:
+        W.free()
+
+
+@pytest.mark.parametrize("values,M,K,N", [("i8", 4096, 1500, 12), ("i8", 512, 512, 64), ("f32", 3000, 768, 9),
+                                          ("f32", 700, 2100, 15), ("i8", 2000, 4000, 200)])
+def test_sliced_copy_built_once_it_pays(ctx, values, M, K, N):
+    """An int8 weight, and a float32 one on 9 to 15 columns: the first product
+    reads the CSR in place (nothing is allocated), a later one builds the
+    sliced-ELL copy, once, and strict products have the oracle's bits on both
+    sides; 16 columns of the float32 weight build theirs at once."""
+    ip, ix, q, sc = workloads.csr_int8_lognormal(M, K, 0.1, 0.5, 0.02, seed=M + N)
+    vals = workloads.dequant_rows(ip, q, sc)
+    X = workloads.dense_normal((K, N), 1.0, seed=N)
+    R = O.orc_csr_spmm(M, K, ip, ix, vals, X)
+    for mode in ("strict", "fast"):
+        W = ctx.csr_upload(M, K, ip, ix, vals) if values == "f32" else ctx.csr_upload(M, K, ip, ix, q, row_scales=sc)
+        b, grew = W.device_bytes(), []
+        for i in range(60):
+            Y = W.spmm(X, mode=mode)
+            assert np.array_equal(bits(Y), bits(R)) if mode == "strict" else close_normwise(Y, R), (mode, i)
+            if W.device_bytes() != b:
+                grew.append(i)
+                b = W.device_bytes()
+        say(f"{values} {M}x{K} N={N} {mode}: copy built by product {grew}")
+        assert len(grew) == 1 and grew[0] > 0
+        W.free()
+    if values == "f32":
+        W = ctx.csr_upload(M, K, ip, ix, vals)
+        b = W.device_bytes()
+        X = workloads.dense_normal((K, 16), 1.0, seed=1)
+        assert np.array_equal(bits(W.spmm(X)), bits(O.orc_csr_spmm(M, K, ip, ix, vals, X)))
+        assert W.device_bytes() > b
         W.free()
