@@ -162,7 +162,8 @@ int pfr_csr_info(const pfr_csr* w, int64_t* M, int64_t* K, int64_t* nnz);
  * stream.  The sliced-ELL copy of an int8 weight, or for 9 to 15 columns, is
  * built later: by the product at which the time lost without it, as estimated,
  * comes to three quarters of the build's (the first or second for long rows
- * and many columns, one after tens for short rows and few).
+ * and many columns, one after tens for short rows and few); without the
+ * memory for it, such products go on reading the CSR in place.
  * While that stream is being captured into a graph, and in
  * pfr_gemm_csr_act_noalloc_dev, nothing is built and a product without its
  * copy runs a kernel that reads the CSR in place (same results in strict

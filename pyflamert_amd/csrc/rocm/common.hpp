@@ -20,6 +20,11 @@ struct Error : std::runtime_error {
     Error(int c, const std::string& m) : std::runtime_error(m), code(c) {}
 };
 
+// No device memory for an allocation: the caller may go on without it.
+struct OutOfMemory : Error {
+    using Error::Error;
+};
+
 void set_last_error(const std::string& msg);
 void clear_last_error();
 

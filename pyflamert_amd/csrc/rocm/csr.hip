@@ -36,7 +36,12 @@ T* dev_alloc_copy(const T* host, int64_t count, hipStream_t s) {
 template <class T>
 T* dev_alloc(int64_t count) {
     void* p = nullptr;
-    PFR_HIP(hipMalloc(&p, sizeof(T) * (size_t)(count > 0 ? count : 1)));
+    const hipError_t e = hipMalloc(&p, sizeof(T) * (size_t)(count > 0 ? count : 1));
+    if (e == hipErrorOutOfMemory) {
+        (void)hipGetLastError();  // or the next launch check finds it
+        throw pfr::OutOfMemory(PFR_ERR_HIP, std::string("hipMalloc: ") + hipGetErrorString(e));
+    }
+    PFR_HIP(e);
     return static_cast<T*>(p);
 }
 

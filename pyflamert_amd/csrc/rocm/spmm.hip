@@ -2484,7 +2484,9 @@ int64_t sell_saving_ns(const pfr_ctx* ctx, const pfr_csr* W, int64_t N, bool fas
 // copy is built when they come to three quarters of its cost: a handle used a few
 // times does not pay for it (the first product of the 11008 x 4096 weight above on
 // 12 columns takes 126 us strict and 118 fast instead of 1051 and 1180), and one
-// used often has lost no more than about the build's time without it.
+// used often has lost no more than about the build's time without it.  Where
+// there is no memory for the copy, such products stay in place and add up anew
+// (an int8 weight of 3 bytes a nonzero may be there only because 8 more are not).
 constexpr int64_t kSellAtOnceN = 16;
 void ensure_copies(const pfr_ctx* ctx, const pfr_csr* W, int64_t N, bool fast, bool strided) {
     const uint32_t pending = W->pending.load(std::memory_order_acquire);
@@ -2496,7 +2498,13 @@ void ensure_copies(const pfr_ctx* ctx, const pfr_csr* W, int64_t N, bool fast, b
     else if (sell != 0) {
         auto& owed = const_cast<pfr_csr*>(W)->sell_owed[fast ? 1 : 0];
         const int64_t saving = std::max<int64_t>(0, sell_saving_ns(ctx, W, N, fast, strided));
-        if (4 * (owed.fetch_add(saving) + saving) >= 3 * sell_build_ns(W, fast)) need |= sell;
+        if (4 * (owed.fetch_add(saving) + saving) >= 3 * sell_build_ns(W, fast)) {
+            try {
+                pfr::csr_build_copies(const_cast<pfr_csr*>(W), sell);
+            } catch (const pfr::OutOfMemory&) {
+                owed.store(0);
+            }
+        }
     }
     if ((pending & need) != 0) pfr::csr_build_copies(const_cast<pfr_csr*>(W), need);
 }

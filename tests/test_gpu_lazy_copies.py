@@ -310,3 +310,76 @@ def test_sliced_copy_built_once_it_pays(ctx, values, M, K, N):
         assert np.array_equal(bits(W.spmm(X)), bits(O.orc_csr_spmm(M, K, ip, ix, vals, X)))
         assert W.device_bytes() > b
         W.free()
+
+
+# hipMalloc that fails with hipErrorOutOfMemory above `limit` bytes.
+NO_MEMORY_C = """
+#include <stddef.h>
+static int (*real)(void**, size_t);
+static size_t limit = (size_t)-1;
+static int refused;
+void set_real(void* f) { real = (int (*)(void**, size_t))f; }
+void set_limit(size_t n) { limit = n; }
+int times_refused(void) { return refused; }
+int hipMalloc(void** p, size_t n) {
+    if (!real) return 3; /* hipErrorNotInitialized */
+    if (n <= limit) return real(p, n);
+    ++refused;
+    *p = 0;
+    return 2; /* hipErrorOutOfMemory */
+}
+"""
+
+NO_MEMORY_PY = """
+import ctypes, re, sys
+shim = ctypes.CDLL(sys.argv[1], mode=ctypes.RTLD_GLOBAL)  # ahead of the HIP runtime, for this process
+shim.set_limit.argtypes = [ctypes.c_size_t]
+sys.path.insert(0, sys.argv[2])
+import numpy as np, torch
+from oracle import oracle as O
+from pyflamert_amd import rocm, workloads
+hip = re.search(r"(/\\S*libamdhip64\\S*)", open("/proc/self/maps").read()).group(1)
+shim.set_real(ctypes.cast(ctypes.CDLL(hip).hipMalloc, ctypes.c_void_p))
+ctx = rocm.Context(0)
+M, K = 4096, 2000
+ip, ix, q, sc = workloads.csr_int8_lognormal(M, K, 0.2, 0.5, 0.02, seed=47)
+vals = workloads.dequant_rows(ip, q, sc)
+for values, N in (("i8", 64), ("f32", 12)):
+    X = workloads.dense_normal((K, N), 1.0, seed=N)
+    R = O.orc_csr_spmm(M, K, ip, ix, vals, X)
+    W = ctx.csr_upload(M, K, ip, ix, vals) if values == "f32" else ctx.csr_upload(M, K, ip, ix, q, row_scales=sc)
+    b = W.device_bytes()
+    W.spmm(X)  # the context's staging buffers
+    assert W.device_bytes() == b
+    shim.set_limit(1 << 20)
+    before = shim.times_refused()
+    for i in range(40):
+        assert np.array_equal(W.spmm(X).view(np.uint32), R.view(np.uint32)), (values, i)
+        assert np.abs(W.spmm(X, mode="fast") - R).max() <= 1e-5 * np.abs(R).max(), (values, i)
+    assert W.device_bytes() == b
+    refused = shim.times_refused() - before
+    assert 2 <= refused < 60, refused  # tried, in both modes, and not by every product
+    shim.set_limit(ctypes.c_size_t(-1).value)
+    for i in range(40):
+        assert np.array_equal(W.spmm(X).view(np.uint32), R.view(np.uint32)), (values, i)
+    assert W.device_bytes() > b
+    print(values, "copies refused", refused, "times, built when there was memory", flush=True)
+"""
+
+
+def test_no_memory_for_a_copy(ctx, tmp_path):
+    """Where the sliced-ELL copy cannot be allocated, the products that did
+    without it before stay in place, with the same bits, and build it once
+    there is memory.  (A process of its own, whose hipMalloc refuses large
+    requests from the host's side; the GPU's memory stays as it is.)"""
+    import os
+    import subprocess
+
+    (tmp_path / "no_memory.c").write_text(NO_MEMORY_C)
+    shim = str(tmp_path / "no_memory.so")
+    subprocess.run(["gcc", "-O1", "-shared", "-fPIC", "-o", shim, str(tmp_path / "no_memory.c")], check=True)
+    root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+    say("products without memory for a copy, in a child process")
+    r = subprocess.run([sys.executable, "-c", NO_MEMORY_PY, shim, root], capture_output=True, text=True, timeout=100)
+    say(r.stdout, r.stderr[-2000:])
+    assert r.returncode == 0 and r.stdout.count("built when there was memory") == 2
