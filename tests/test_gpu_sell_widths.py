@@ -128,3 +128,35 @@ def test_nonfinite_rule_in_kernel(ctx, M, K, N, alpha, act):
         ok = ~np.isnan(R)
         assert np.array_equal(Y[ok].view(np.uint32), R[ok].view(np.uint32))
     W.free()
+
+
+@pytest.mark.parametrize("values", ["f32", "i8"])
+def test_rows_that_repeat_columns(ctx, values):
+    """Rows that list a column several times: where one has more entries in a
+    chunk than the chunk has columns, the fast copy keeps storage order."""
+    M, K, N = 40, 2100, 17
+    rng = np.random.default_rng(90)
+    cols = []
+    for r in range(M):
+        n = 1500 if r in (3, 20) else int(rng.integers(0, 300))
+        c = rng.integers(0, 1000 if n == 1500 else K, n)  # more than 1024 entries in columns 0 .. 999
+        cols.append(np.sort(c))
+    ip = np.concatenate([[0], np.cumsum([len(c) for c in cols])])
+    ix = np.concatenate(cols)
+    q = rng.integers(1, 100, len(ix)).astype(np.int8)
+    sc = rng.uniform(0.001, 0.002, M).astype(np.float32)
+    vals = workloads.dequant_rows(ip, q, sc)
+    X = workloads.dense_normal((K, N), 1.0, seed=91)
+    W = ctx.csr_upload(M, K, ip, ix, vals) if values == "f32" else ctx.csr_upload(M, K, ip, ix, q, row_scales=sc)
+    build_copies(W, K)
+    print(f"rows that repeat columns: {values}", flush=True)
+    R = O.orc_csr_spmm(M, K, ip, ix, vals, X)
+    assert np.array_equal(W.spmm(X, mode="strict").view(np.uint32), R.view(np.uint32))
+    F = W.spmm(X, mode="fast").astype(np.float64)
+    exact, mag = np.zeros((M, N)), np.zeros((M, N))
+    for r in range(M):
+        v, x = vals[ip[r]:ip[r + 1], None].astype(np.float64), X[ix[ip[r]:ip[r + 1]]].astype(np.float64)
+        exact[r], mag[r] = (v * x).sum(0), np.abs(v * x).sum(0)
+    g = (np.diff(ip)[:, None] + 2) * 2.0 ** -24
+    assert (np.abs(F - exact) <= g / (1 - g) * mag + 1e-30).all()
+    W.free()
