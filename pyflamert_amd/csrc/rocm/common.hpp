@@ -279,7 +279,7 @@ struct pfr_csr {
     // hold whole records of four entries and then one spare record (padding
     // entries: value 0, column K).
     int2* mp_wave = nullptr;
-    int4* mp_wmeta = nullptr;  // [Q] the rows each wave shares within its workgroup (set_merge)
+    int4* mp_wmeta = nullptr;  // [Q] the rows each wave shares within its workgroup (plan_merge in csr.hip)
     int4* mp_grp = nullptr;
     unsigned long long* mp_xchg = nullptr;
     float* mp_carry = nullptr;

@@ -2572,7 +2572,7 @@ void gemm_dev(pfr_ctx* ctx, const float* A, int64_t Mb, int64_t K, int transA, c
         // stage through registers, more slowly than the direct-to-LDS copy of
         // a transposed A, so this pays off when the launch runs in one round
         // (every workgroup stages once, side by side): 768 x 768, 20 %, at 1024
-        // tokens 22.4 -> 17.2 us; 3072 x 768 (three rounds) 46.0 -> 53.8 us.  (A
+        // tokens 22.4 -> 16.9 us; 3072 x 768 (three rounds) 46.0 -> 53.8 us.  (A
         // weight of one chunk gains in two rounds too, 768 x 768 at 2048 tokens
         // 34.4 -> 31.1, and loses 6 % on 16 to 64 tokens, 10.6 -> 11.3.)
         launch_spmm(ctx, BT, A, Mb, K, Y, 1, Nf, C, c_size, beta, mode == PFR_MODE_FAST, act, false, true, alpha);
