@@ -143,8 +143,8 @@ int pfr_csr_from_dense_dev(pfr_ctx* ctx, const float* dense, int64_t rows,
  * the CSR does not store (inf * 0 = NaN), which sparse_matmul
  * (sparse_tensor.cpp:473-519) skips.  Builds a bitmap of the stored entries
  * (M x ceil(K / 64) words); from then on every product through the handle
- * is followed by a fix-up pass over the activations that writes NaN (through
- * the bias and activation epilogue) where an inf activation meets an
+ * is followed by a fix-up pass over the activations, or applies it itself, that
+ * writes NaN (through the bias and activation epilogue) where an inf activation meets an
  * unstored weight or a NaN activation meets any weight of an output.  For
  * finite activations results are unchanged.  Idempotent. */
 int pfr_csr_dense_semantics(pfr_csr* w);

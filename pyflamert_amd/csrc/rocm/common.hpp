@@ -68,12 +68,12 @@ __device__ __forceinline__ int32_t f2i_trunc_x86(float r) {
 
 // cpu_gelu (activation.cpp:249-256): 0.5 v (1 + tanh(u)) with the reference's
 // u, as v / (1 + exp(-2 u)), the same function: 0.5 (1 + tanh(u)) is the
-// logistic function of 2 u.  It costs about half of the device's tanhf, which
+// logistic function of 2 u.  It costs less than the device's tanhf, which
 // with a division per bias index took a quarter of the 3072 x 768 product's
 // launch on 1024 tokens (57 -> 44 us with the other epilogue change and one LDS
 // buffer, see k_spmm_sell).  d + de is 1 + e exactly where e < 2^24, and the
 // quotient v r is corrected by its remainder, so expf's error (halved or less
-// by the sum) and u's are all that is left: rms error against 64 bits 0.31 -
+// by the sum) and u's are all that is left: rms error against 64 bits 0.29 -
 // 0.36 ulp on [-0.1, 3], where the reference's sequence with the device's
 // tanhf has 0.36 - 0.50 and the plain v * rcp(1 + e) 0.52 - 0.65.  Far below
 // zero the reference's 1 + tanhf(u) cancels (an ulp of 1 in it; -0 from about
@@ -288,7 +288,7 @@ struct pfr_csr {
     // Stored-entry bitmap (set by pfr_csr_dense_semantics): bit k % 64 of
     // pattern[r * pattern_nw + k / 64] is set when row r stores column k.
     // While it is set, every product through the handle is followed by the
-    // non-finite fix-up, which gives the dense kernels' results where an inf
+    // non-finite fix-up, or applies its rule itself (k_spmm_sell), which gives the dense kernels' results where an inf
     // or NaN activation meets a weight the CSR does not store (a zero).
     uint64_t* pattern = nullptr;
     int64_t pattern_nw = 0;
