@@ -1720,7 +1720,8 @@ constexpr SmallTile kSmallTiles[] = {{1, 1, 8, 3500, 870, 24},
 // row-major; then a tile narrower than the rows reads pieces of lines (4096 x
 // 4096 int8 on 128 columns: 64 x 32 tiles 13.0 us, against 7.3 after a transpose
 // of 4), so only tiles as wide as the rows, or the widest, are taken, and the
-// widest's steps take 170 ns.  Every workgroup reads its columns of X anew, so
+// widest's steps take 170 ns (bf16: 140 where two workgroups share a CU; 4096 x
+// 11008 on 320 columns 51 us, against 58 from the transpose).  Every workgroup reads its columns of X anew, so
 // steps slow down as X outgrows an XCD's 4 MiB L2.
 int small_tile(const pfr_ctx* ctx, const pfr_sp24* W, int64_t N, int64_t steps, bool in_place, int64_t* ns) {
     const bool bf = W->dtype == PFR_BF16;
@@ -1733,7 +1734,7 @@ int small_tile(const pfr_ctx* ctx, const pfr_sp24* W, int64_t N, int64_t steps, 
         if (in_place && t.nb < 4 && 16 * t.nb < N) continue;
         const int64_t wgs = (W->M + 16 * t.rb - 1) / (16 * t.rb) * ((N + 16 * t.nb - 1) / (16 * t.nb));
         const int64_t per_cu = (wgs + ctx->num_cu - 1) / ctx->num_cu;
-        const double step = in_place && t.nb == 4 ? 170 : t.step;
+        const double step = in_place && t.nb == 4 ? (bf && per_cu == 2 ? 140 : 170) : t.step;
         const int64_t e = t.start + per_cu * (t.each + (int64_t)((double)steps * step * slow));
         if (e < *ns) *ns = e, best = i;
     }

@@ -51,7 +51,7 @@ def small_tile_rule():
     tiles = [tuple(map(int, t.split(","))) for t in re.findall(r"\{([\d, ]+)\}", table)]
     assert len(tiles) == 5
     for line in ("const double slow = 1 + (bf ? 0.1 : 0.25) * std::max(0.0, spill);",
-                 "const double step = in_place && t.nb == 4 ? 170 : t.step;",
+                 "const double step = in_place && t.nb == 4 ? (bf && per_cu == 2 ? 140 : 170) : t.step;",
                  "const double rounds = full > 1 ? 0.75 * (double)full + 0.25 * (double)tiles / ctx->num_cu : 1;",
                  "std::min<int64_t>(380 + 9 * busy / 2, 600)", "(xrow ? 430 + 7 * busy / 10 : 500 + 14 * busy / 10)",
                  "const double scale = W->dtype == PFR_I8 && !xrow && whole ? 0.85 : 1;",
@@ -67,7 +67,9 @@ def small_tile_rule():
             if in_place and nb < 4 and 16 * nb < N:
                 continue
             n = up(up(M, 16 * rb) * up(N, 16 * nb), CUS)
-            t = start + n * (each + int(steps * (170 if in_place and nb == 4 else step) * slow))
+            if in_place and nb == 4:
+                step = 140 if size == 2 and n == 2 else 170
+            t = start + n * (each + int(steps * step * slow))
             if best is None or t < best[0]:
                 best = (t, i)
         return best
